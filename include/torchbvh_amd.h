@@ -218,6 +218,17 @@ int tbvh_knn_accel_grid_positions(const void* accel, const float* node_aabbs,
                                   int64_t* out_indices, float* out_distances,
                                   float* out_positions, void* workspace,
                                   size_t workspace_bytes, void* stream);
+/* tbvh_knn_accel for calls of few queries: one wave per query over the
+ * implicit tree's boxes (node_aabbs, as the build wrote them) and the accel's
+ * points.  The same results as tbvh_knn_accel, or, with `spatial` nonzero,
+ * tbvh_knn_accel_spatial; with source_points (nullable) also
+ * tbvh_knn_accel_positions' rows.  No workspace. */
+int tbvh_knn_accel_wave(const void* accel, const float* node_aabbs, int64_t num_real_nodes,
+                        const float* queries, const int64_t* order, int64_t B, int64_t M,
+                        int64_t num_leaves, int D, int k, int spatial,
+                        const float* source_points, int source_cols,
+                        int64_t* out_indices, float* out_distances, float* out_positions,
+                        void* stream);
 int tbvh_knn_accel_ragged_positions(const void* accel, const int64_t* point_offsets,
                                     int64_t total_points, const float* queries,
                                     const int64_t* query_offsets, const int64_t* order,

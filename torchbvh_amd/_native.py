@@ -119,6 +119,9 @@ def _declare(L) -> None:
     L.tbvh_knn_accel_grid_positions.argtypes = (
         [_vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _int, _int, _vp, _int, _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp]
     )
+    L.tbvh_knn_accel_wave.argtypes = (
+        [_vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _int, _int, _int, _vp, _int, _vp, _vp, _vp, _vp]
+    )
     L.tbvh_knn_accel_ragged_positions.argtypes = (
         [_vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _int, _int, _vp, _int, _vp, _vp, _vp, _vp]
     )
@@ -133,7 +136,7 @@ def _declare(L) -> None:
         "tbvh_accel_workspace_size", "tbvh_accel_build", "tbvh_accel_build_ragged",
         "tbvh_knn_accel", "tbvh_knn_accel_ragged", "tbvh_knn_spatial", "tbvh_knn_accel_spatial",
         "tbvh_knn_accel_grid_workspace_size", "tbvh_knn_accel_grid", "tbvh_knn_accel_grid_spatial",
-        "tbvh_knn_accel_positions", "tbvh_knn_accel_grid_positions", "tbvh_knn_accel_ragged_positions",
+        "tbvh_knn_accel_positions", "tbvh_knn_accel_grid_positions", "tbvh_knn_accel_ragged_positions", "tbvh_knn_accel_wave",
         "tbvh_sort_routed_queries_workspace_size", "tbvh_sort_routed_queries",
         "tbvh_knn_routed_spatial", "tbvh_knn_accel_routed_spatial",
         "tbvh_knn_accel_routed_grid_workspace_size", "tbvh_knn_accel_routed_grid_spatial",
@@ -237,6 +240,28 @@ MAX_ACCEL_CLOUD = 1 << 28
 # search (tbvh_knn_accel_grid); below it its three extra launches cost more
 # than it saves.
 GRID_MIN_QUERIES = 1 << 17
+
+# Batched accel k-NN calls of at most this many queries search with one wave
+# per query (tbvh_knn_accel_wave); the traversal takes one query per lane and
+# its time hardly depends on the number of queries until they fill the chip.
+# Measured (call, wave / traversal, us).  3-D, uniform: 50,000 points, 1,000
+# queries k = 8 23 / 73; 10,000 points, 8,000 queries k = 4 29 / 58; 300,000
+# points, 16,000 queries k = 4 98 / 97, k = 16 129 / 147, 32,000 queries k = 16
+# 210 / 151; clustered or surface clouds with queries away from the points gain
+# most (50,000 on a surface, 16,000 queries k = 16 119 / 913).  2-D boxes
+# overlap less, so the traversal is shorter: 10,000 points, 8,000 queries k =
+# 4 23 / 31, 16,000 34 / 32; 300,000 points, 4,000 queries k = 4 40 / 41, 8,000
+# 59 / 40.
+WAVE_MAX_QUERIES = 1 << 14          # 3-D
+WAVE_MAX_QUERIES_2D = 1 << 13       # 2-D, clouds of at most WAVE_2D_CLOUD points
+WAVE_MAX_QUERIES_2D_LARGE = 1 << 12
+WAVE_2D_CLOUD = 1 << 16
+
+
+def _wave_limit(dim: int, num_leaves: int) -> int:
+    if dim == 3:
+        return WAVE_MAX_QUERIES
+    return WAVE_MAX_QUERIES_2D if num_leaves <= WAVE_2D_CLOUD else WAVE_MAX_QUERIES_2D_LARGE
 
 
 @functools.lru_cache(maxsize=256)
@@ -804,7 +829,12 @@ class _NativeOps:
         with torch.cuda.device(dev):
             grid = (accel is not None and B * M > GRID_MIN_QUERIES
                     and _grid_workspace_size(B, M, int(num_leaves), int(dim), int(k)) > 0)
-            if fused and grid and not spatial:
+            if accel is not None and B * M <= _wave_limit(int(dim), int(num_leaves)):
+                _check(L.tbvh_knn_accel_wave(
+                    _ptr(accel), _ptr(node_aabbs), int(num_real_nodes), _ptr(query_points), _ptr(query_order),
+                    B, M, int(num_leaves), int(dim), int(k), int(spatial), _ptr(source_points) if fused else None,
+                    C if fused else 0, _ptr(indices), _ptr(distances), _ptr(positions), _stream(dev)))
+            elif fused and grid and not spatial:
                 # The cell-block search with the neighbour rows (the same
                 # rows as tbvh_knn_accel_positions).
                 need = _grid_workspace_size(B, M, int(num_leaves), int(dim), int(k))

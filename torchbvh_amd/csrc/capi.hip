@@ -954,7 +954,8 @@ static int knn_accel_batched(const char* op, const void* accel, const float* que
                              int k, bool spatial, int64_t* out_indices, float* out_distances,
                              void* stream_ptr, const float* source_points = nullptr, int source_cols = 0,
                              float* out_positions = nullptr, const float* node_aabbs = nullptr,
-                             int64_t num_real_nodes = 0, void* ws = nullptr, size_t ws_bytes = 0) {
+                             int64_t num_real_nodes = 0, void* ws = nullptr, size_t ws_bytes = 0,
+                             bool wave = false) {
     if (int r = check_dim(op, D)) return r;
     if (!supported_k(k)) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: k must be 4, 8, or 16 (32 is also supported), got %d", op, k);
     if (B < 1 || M < 0) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: need B >= 1 and M >= 0", op);
@@ -985,11 +986,19 @@ static int knn_accel_batched(const char* op, const void* accel, const float* que
     a.source_cols = source_cols;
     a.out_positions = out_positions;
     const int level = ws ? grid_level(num_leaves, D, k) : 0;
-    if (level > 0) {
+    if (level > 0 || wave) {
         if (!node_aabbs) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: null node_aabbs", op);
         if (num_real_nodes != tree::real_node_count(static_cast<int>(num_leaves))) {
             return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: num_real_nodes does not match num_leaves", op);
         }
+    }
+    if (wave) {
+        a.node_aabbs = node_aabbs;
+        a.num_real_nodes = static_cast<int32_t>(num_real_nodes);
+        TBVH_TRY(op, launch_knn_wave(a, D, k, static_cast<hipStream_t>(stream_ptr)));
+        return ok();
+    }
+    if (level > 0) {
         if (!aligned(ws)) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: workspace must be %zu-byte aligned", op, kAlign);
         const size_t need = grid_workspace_bytes(B, B * M, level, D);
         if (ws_bytes < need) {
@@ -1120,6 +1129,19 @@ int tbvh_knn_accel_grid_positions(const void* accel, const float* node_aabbs, in
     return knn_accel_batched(op, accel, queries, order, B, M, num_leaves, D, k, false, out_indices, out_distances,
                              stream_ptr, source_points, source_cols, out_positions, node_aabbs, num_real_nodes,
                              ws, ws_bytes);
+}
+
+int tbvh_knn_accel_wave(const void* accel, const float* node_aabbs, int64_t num_real_nodes, const float* queries,
+                        const int64_t* order, int64_t B, int64_t M, int64_t num_leaves, int D, int k, int spatial,
+                        const float* source_points, int source_cols, int64_t* out_indices, float* out_distances,
+                        float* out_positions, void* stream_ptr) {
+    const char* op = "tbvh_knn_accel_wave";
+    if (source_points || out_positions) {
+        if (int r = check_positions(op, source_points, source_cols, out_positions)) return r;
+    }
+    return knn_accel_batched(op, accel, queries, order, B, M, num_leaves, D, k, spatial != 0, out_indices,
+                             out_distances, stream_ptr, source_points, source_cols, out_positions, node_aabbs,
+                             num_real_nodes, nullptr, 0, true);
 }
 
 int tbvh_knn_accel_ragged_positions(const void* accel, const int64_t* point_offsets, int64_t total_points,

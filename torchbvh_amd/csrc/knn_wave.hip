@@ -1,0 +1,338 @@
+// Exact k-NN with one wave per query, for calls of few queries.
+//
+// A traversal with one query per lane (knn.hip) is a chain of about 140
+// dependent steps per wave whatever the call's size: 1,000 queries are 16
+// waves on a chip of 256 CUs, and the call takes that chain's latency.  Here
+// a wave's 64 lanes work on one query: a step tests 64 boxes of the implicit
+// tree or 64 points at once, and the chain is about ten steps.
+//
+// Boxes.  The implicit tree's node at depth L - s covers 2^s consecutive
+// Morton-ordered points, and the nodes of a level are consecutive rows, so
+// the boxes of 64 sibling runs are one contiguous read.  The wave descends
+// six levels at a time: runs of 16 points ("blocks") at the bottom, then of
+// 1,024, 65,536, ..., up to a top level of at most 64 nodes.  These boxes
+// overlap more than the radix tree's (a run may straddle a large Morton
+// cell's border), which costs 64-wide tests little.
+//
+// List.  One key per lane, ascending over the lanes: the 64 smallest keys
+// seen (the first K are the result).  The first four blocks (64 points,
+// nearest first) fill it by one bitonic sort over the lanes; later points
+// below the k-th key wait in LDS and are merged 64 at a time.  Keys and
+// distances are the traversal's, so the result is the same k smallest
+// (distance, index) pairs, bit for bit; a box is skipped only when its
+// distance exceeds the k-th distance.
+//
+// Bound: a lone query takes the chain of dependent reads and exchanges (about
+// 15 us for 50,000 points); many, about 1,500 issue slots each.  Measured, call
+// time against the traversal: 1,000 queries of 50,000 3-D points at k = 8
+// 73 -> 23 us, 10,000 of 10,000 at k = 4 64 -> 31 us (kernel); which calls take
+// it: WAVE_MAX_QUERIES in _native.py.
+#include "knn_common.hpp"
+
+namespace tbvh {
+namespace {
+
+constexpr int kBlockBits = 4;   // points per block: 16
+constexpr int kFanBits = 6;     // levels per step: 64 children
+constexpr int kMergeAt = 32;    // pending candidates that trigger a merge
+
+template <int kCtrl>
+__device__ __forceinline__ uint64_t dpp_key(uint64_t k) {
+    const int lo = __builtin_amdgcn_mov_dpp(static_cast<int>(static_cast<uint32_t>(k)), kCtrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(static_cast<int>(static_cast<uint32_t>(k >> 32)), kCtrl, 0xf, 0xf, true);
+    return (static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo);
+}
+constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kXor3 = 0x1B;                // quad_perm
+constexpr int kXor7 = 0x141, kXor15 = 0x140, kRor8 = 0x128;            // row mirrors, rotate by half a row
+
+// Keys of the two 16-lane rows (kRow16) or two wave halves of each pair, as
+// (even / low one's, odd / high one's) in every lane.
+template <bool kRow16>
+__device__ __forceinline__ void pair_keys(uint64_t k, uint64_t& even, uint64_t& odd) {
+    const uint32_t lo = static_cast<uint32_t>(k), hi = static_cast<uint32_t>(k >> 32);
+    const auto l = kRow16 ? __builtin_amdgcn_permlane16_swap(lo, lo, false, false)
+                          : __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = kRow16 ? __builtin_amdgcn_permlane16_swap(hi, hi, false, false)
+                          : __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    even = (static_cast<uint64_t>(h[0]) << 32) | l[0];
+    odd = (static_cast<uint64_t>(h[1]) << 32) | l[1];
+}
+
+// This lane's key becomes the smaller (lane bit kBit clear) or larger of it
+// and `other`.
+template <int kBit>
+__device__ __forceinline__ uint64_t keep(uint64_t k, uint64_t other) {
+    const uint64_t mn = key_min(k, other), mx = key_max(k, other);
+    return (lane_id() & kBit) ? mx : mn;
+}
+
+// Compare-exchange with the lane kStride away.
+template <int kStride>
+__device__ __forceinline__ uint64_t exchange(uint64_t k) {
+    if constexpr (kStride == 1) return keep<1>(k, dpp_key<kXor1>(k));
+    else if constexpr (kStride == 2) return keep<2>(k, dpp_key<kXor2>(k));
+    else if constexpr (kStride == 4) return keep<4>(k, dpp_key<kXor3>(dpp_key<kXor7>(k)));
+    else if constexpr (kStride == 8) return keep<8>(k, dpp_key<kRor8>(k));
+    else {
+        uint64_t even, odd;
+        pair_keys<kStride == 16>(k, even, odd);
+        return keep<kStride>(even, odd);
+    }
+}
+
+// The key of lane 31 - l (of its half) and of lane 63 - l.
+__device__ __forceinline__ uint64_t reversed32(uint64_t k) {
+    uint64_t even, odd;
+    pair_keys<true>(dpp_key<kXor15>(k), even, odd);
+    return (lane_id() & 16) ? even : odd;
+}
+__device__ __forceinline__ uint64_t reversed64(uint64_t k) {
+    uint64_t even, odd;
+    pair_keys<false>(reversed32(k), even, odd);
+    return (lane_id() & 32) ? even : odd;
+}
+
+// Bitonic sequence over the 64 lanes -> ascending.
+__device__ __forceinline__ uint64_t clean64(uint64_t k) {
+    k = exchange<32>(k);
+    k = exchange<16>(k);
+    k = exchange<8>(k);
+    k = exchange<4>(k);
+    k = exchange<2>(k);
+    return exchange<1>(k);
+}
+
+// Ascending over the 64 lanes (bitonic sort whose merges start with the
+// second run reversed, so every exchange is ascending).
+__device__ __forceinline__ uint64_t sort64(uint64_t k) {
+    k = keep<1>(k, dpp_key<kXor1>(k));
+    k = keep<2>(k, dpp_key<kXor3>(k));
+    k = exchange<1>(k);
+    k = keep<4>(k, dpp_key<kXor7>(k));
+    k = exchange<2>(k);
+    k = exchange<1>(k);
+    k = keep<8>(k, dpp_key<kXor15>(k));
+    k = exchange<4>(k);
+    k = exchange<2>(k);
+    k = exchange<1>(k);
+    k = keep<16>(k, reversed32(k));
+    k = exchange<8>(k);
+    k = exchange<4>(k);
+    k = exchange<2>(k);
+    k = exchange<1>(k);
+    k = keep<32>(k, reversed64(k));
+    k = exchange<16>(k);
+    k = exchange<8>(k);
+    k = exchange<4>(k);
+    k = exchange<2>(k);
+    return exchange<1>(k);
+}
+
+// Smallest value over the wave.
+__device__ __forceinline__ uint32_t wave_least(uint32_t v) {
+    const auto step = [&](auto shifted) { v = min(v, static_cast<uint32_t>(shifted)); };
+    step(__builtin_amdgcn_update_dpp(-1, static_cast<int>(v), 0x111, 0xf, 0xf, false));  // row_shr:1
+    step(__builtin_amdgcn_update_dpp(-1, static_cast<int>(v), 0x112, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(-1, static_cast<int>(v), 0x114, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(-1, static_cast<int>(v), 0x118, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(-1, static_cast<int>(v), 0x142, 0xa, 0xf, false));  // row_bcast:15
+    step(__builtin_amdgcn_update_dpp(-1, static_cast<int>(v), 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
+}
+
+// Lane (set in `mask`) with the smallest distance, ties within 2^-17 of each
+// other to the lower lane.
+__device__ __forceinline__ int nearest_lane(float d, uint64_t mask) {
+    const bool in = (mask >> lane_id()) & 1ull;
+    const uint32_t k = in ? (__float_as_uint(d) & ~63u) | static_cast<uint32_t>(lane_id()) : 0xffffffffu;
+    return static_cast<int>(wave_least(k) & 63u);
+}
+
+template <int D, int K>
+struct WaveQuery {
+    const float* nodes;   // this cloud's rows of 2 * D floats
+    const float4* pts;    // this cloud's Morton-ordered points
+    int n, L, vl, bl;     // points, leaf level, virtual leaves, block level
+    float q[D];
+    uint64_t* pend;       // candidates waiting for a merge (128 keys of LDS)
+    int waiting;          // how many (wave-uniform)
+    bool filled;          // the first blocks are in the list
+    uint64_t list;        // this lane's key, ascending over the lanes
+    uint64_t kth;         // key of lane K - 1 (wave-uniform)
+    float worst;          // its distance
+
+    __device__ __forceinline__ void set_kth() {
+        const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(list), K - 1);
+        const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(list >> 32), K - 1);
+        kth = (static_cast<uint64_t>(hi) << 32) | lo;
+        worst = __uint_as_float(hi);
+    }
+
+    __device__ __forceinline__ void merge() {
+        __builtin_amdgcn_wave_barrier();
+        for (int base = 0; base < waiting; base += kWave) {
+            const uint64_t k = base + lane_id() < waiting ? pend[base + lane_id()] : kEmptyKey;
+            list = clean64(key_min(list, reversed64(sort64(k))));
+        }
+        __builtin_amdgcn_wave_barrier();
+        waiting = 0;
+        set_kth();
+    }
+
+    // Distance from the query to node `i` of `level`; +inf past the level's
+    // real nodes.
+    __device__ __forceinline__ float node_distance(int level, int i) const {
+        const int real = tree::real_at_level(vl, L, level);
+        if (i >= real) return INFINITY;
+        const int row0 = tree::level_first(level) - tree::virtual_above(vl, L, level);
+        float box[2 * D];
+        const float* b = nodes + static_cast<int64_t>(row0 + i) * (2 * D);
+#pragma unroll
+        for (int d = 0; d < 2 * D; ++d) box[d] = b[d];
+        return box_distance<D>(q, box);
+    }
+
+    // The points of the blocks first + (bits of mask), `d` each lane's block
+    // distance.
+    __device__ __forceinline__ void scan_blocks(int first, uint64_t mask, float d) {
+        const int bits = L - bl;
+        const int slot = lane_id() & 15;
+        while (mask != 0) {
+            // Four blocks, 16 lanes each: the nearest four while the list is
+            // empty, then in storage order.
+            int mine = -1;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                if (mask != 0) {
+                    const int b = filled ? __ffsll(static_cast<long long>(mask)) - 1 : nearest_lane(d, mask);
+                    mask &= ~(1ull << b);
+                    if ((lane_id() >> 4) == g) mine = first + b;
+                }
+            }
+            const int at = (mine << bits) + slot;
+            const bool valid = mine >= 0 && slot < (1 << bits) && at < n;
+            const float4 p = pts[valid ? at : 0];
+            const float dist = point_distance<D>(q, p);
+            const uint64_t key = valid && dist < kFar ? candidate_key(dist, __float_as_uint(p.w)) : kEmptyKey;
+            if (!filled) {
+                filled = true;
+                list = sort64(key);
+                set_kth();
+            } else {
+                const bool in = key < kth;
+                const uint64_t m = __ballot(in);
+                if (m == 0) continue;
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
+                if (in) pend[waiting + rank] = key;
+                waiting += __popcll(m);
+                if (waiting < kMergeAt) continue;
+                merge();
+            }
+            mask &= __ballot(d <= worst);
+        }
+    }
+
+    // Visits the children (at `level`) of node `parent`, six levels up; the
+    // level is bl - 6 * kBelow.
+    template <int kBelow>
+    __device__ __forceinline__ void expand(int parent) {
+        const int level = bl - kBelow * kFanBits;
+        const int first = parent << kFanBits;
+        const float d = node_distance(level, first + lane_id());
+        uint64_t mask = __ballot(d <= worst && d < INFINITY);
+        if constexpr (kBelow == 0) {
+            scan_blocks(first, mask, d);
+        } else {
+            while (mask != 0) {
+                const int c = nearest_lane(d, mask);
+                expand<kBelow - 1>(first + c);
+                mask &= ~(1ull << c);
+                // The candidates still waiting tighten the bound before the
+                // next run's boxes are read.
+                if (mask != 0 && waiting > 0) merge();
+                mask &= __ballot(d <= worst);
+            }
+        }
+    }
+};
+
+template <int D, int K, int kSteps>
+__global__ __launch_bounds__(kWave) void knn_wave_kernel(KnnArgs a) {
+    __shared__ uint64_t s_pend[kMergeAt + kWave];
+    const int64_t gid = blockIdx.x;
+    const int64_t seg = gid / a.M;
+    const int64_t local = gid - seg * a.M;
+    const int64_t qi = a.order != nullptr ? a.order[gid] : local;
+    if (qi < 0 || qi >= a.M) return;  // a corrupt order never indexes out of range
+    const int64_t row = seg * a.M + qi;
+    const int64_t pstart = seg * a.num_leaves;
+    WaveQuery<D, K> w;
+    w.nodes = a.node_aabbs + seg * a.num_real_nodes * (2 * D);
+    w.pts = static_cast<const float4*>(a.accel) + pstart;
+    w.n = a.num_leaves;
+    w.L = tree::leaf_level(w.n);
+    w.vl = tree::virtual_leaves(w.n);
+    w.bl = w.L > kBlockBits ? w.L - kBlockBits : 0;
+#pragma unroll
+    for (int d = 0; d < D; ++d) w.q[d] = a.queries[row * D + d];
+    w.pend = s_pend;
+    w.waiting = 0;
+    w.filled = false;
+    w.list = kEmptyKey;
+    w.kth = kEmptyKey;
+    w.worst = kFar;
+    w.template expand<kSteps - 1>(0);
+    if (w.waiting > 0) w.merge();
+
+    if (lane_id() < K) {
+        const int64_t out_row = a.spatial_output ? gid : row;
+        const int64_t idx = static_cast<int32_t>(static_cast<uint32_t>(w.list));
+        a.out_indices[out_row * K + lane_id()] = idx;
+        a.out_distances[out_row * K + lane_id()] = __uint_as_float(static_cast<uint32_t>(w.list >> 32));
+        if (a.out_positions != nullptr) {
+            const int C = a.source_cols;
+            float* op = a.out_positions + (out_row * K + lane_id()) * C;
+            const float* src = a.source_points + (pstart + (idx >= 0 ? idx : 0)) * C;
+            for (int c = 0; c < C; ++c) op[c] = idx >= 0 ? src[c] : 0.0f;
+        }
+    }
+}
+
+template <int D, int K>
+void launch_steps(const KnnArgs& a, hipStream_t stream) {
+    const unsigned grid = static_cast<unsigned>(a.total_q);
+    // Wide steps from a top level of at most 64 nodes down to the blocks.
+    const int L = tree::leaf_level(a.num_leaves);
+    const int bl = L > kBlockBits ? L - kBlockBits : 0;
+    const int steps = bl <= kFanBits ? 1 : (bl + kFanBits - 1) / kFanBits;
+    switch (steps) {
+        case 1: knn_wave_kernel<D, K, 1><<<grid, kWave, 0, stream>>>(a); break;
+        case 2: knn_wave_kernel<D, K, 2><<<grid, kWave, 0, stream>>>(a); break;
+        case 3: knn_wave_kernel<D, K, 3><<<grid, kWave, 0, stream>>>(a); break;
+        default: knn_wave_kernel<D, K, 4><<<grid, kWave, 0, stream>>>(a); break;
+    }
+}
+
+template <int D>
+hipError_t launch_k(const KnnArgs& a, int K, hipStream_t stream) {
+    switch (K) {
+        case 4: launch_steps<D, 4>(a, stream); break;
+        case 8: launch_steps<D, 8>(a, stream); break;
+        case 16: launch_steps<D, 16>(a, stream); break;
+        case 32: launch_steps<D, 32>(a, stream); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_knn_wave(const KnnArgs& a, int D, int K, hipStream_t stream) {
+    if (a.total_q == 0) return hipSuccess;
+    // Four steps of six levels and the blocks' four cover 2^28 points.
+    if (a.num_leaves < 1 || a.num_leaves > kMaxAccelCloud) return hipErrorInvalidValue;
+    return D == 3 ? launch_k<3>(a, K, stream) : launch_k<2>(a, K, stream);
+}
+
+}  // namespace tbvh

@@ -442,6 +442,10 @@ struct KnnArgs {
 hipError_t launch_knn(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream);
 hipError_t launch_knn_accel(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream);
 
+// Batched accel k-NN with one wave per query (knn_wave.hip; not routed):
+// reads the accel's points and node_aabbs.
+hipError_t launch_knn_wave(const KnnArgs& a, int D, int K, hipStream_t stream);
+
 // Cell-block k-NN (batched accel, `a` as for launch_knn_accel; spatial
 // output and neighbour rows as there): every cloud's accel points are cut
 // into the level-`level` Morton cells against its root box (row 0 of its
