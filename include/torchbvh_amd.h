@@ -229,6 +229,34 @@ int tbvh_knn_accel_wave(const void* accel, const float* node_aabbs, int64_t num_
                         const float* source_points, int source_cols,
                         int64_t* out_indices, float* out_distances, float* out_positions,
                         void* stream);
+/* tbvh_knn_accel (with `spatial` nonzero, tbvh_knn_accel_spatial; with
+ * source_points, nullable, also tbvh_knn_accel_positions' rows) whose waves
+ * give up their last, slowest queries to a second launch of one wave per
+ * query over node_aabbs (as the build wrote them).  The same results. */
+int tbvh_knn_tail_workspace_size(int64_t total_q, int D, size_t* bytes); /* 0: one launch */
+int tbvh_knn_accel_tail(const void* accel, const float* node_aabbs, int64_t num_real_nodes,
+                        const float* queries, const int64_t* order, int64_t B, int64_t M,
+                        int64_t num_leaves, int D, int k, int spatial,
+                        const float* source_points, int source_cols,
+                        int64_t* out_indices, float* out_distances, float* out_positions,
+                        void* workspace, size_t workspace_bytes, void* stream);
+int tbvh_knn_accel_ragged_tail(const void* accel, const float* node_aabbs,
+                               const int64_t* node_offsets, const int64_t* point_offsets,
+                               int64_t total_points, const float* queries,
+                               const int64_t* query_offsets, const int64_t* order,
+                               int64_t B, int64_t total_q, int D, int k,
+                               const float* source_points, int source_cols,
+                               int64_t* out_indices, float* out_distances, float* out_positions,
+                               void* workspace, size_t workspace_bytes, void* stream);
+/* tbvh_knn_accel_wave for ragged calls. */
+int tbvh_knn_accel_ragged_wave(const void* accel, const float* node_aabbs,
+                               const int64_t* node_offsets, const int64_t* point_offsets,
+                               int64_t total_points, const float* queries,
+                               const int64_t* query_offsets, const int64_t* order,
+                               int64_t B, int64_t total_q, int D, int k,
+                               const float* source_points, int source_cols,
+                               int64_t* out_indices, float* out_distances, float* out_positions,
+                               void* stream);
 int tbvh_knn_accel_ragged_positions(const void* accel, const int64_t* point_offsets,
                                     int64_t total_points, const float* queries,
                                     const int64_t* query_offsets, const int64_t* order,
@@ -440,6 +468,17 @@ int tbvh_knn_accel_routed_spatial(const void* true_accel, const void* false_acce
                                   int64_t true_num_leaves, int64_t false_num_leaves,
                                   int D, int k,
                                   int64_t* out_indices, float* out_distances, void* stream);
+/* tbvh_knn_accel_routed_spatial with the second launch of tbvh_knn_accel_tail
+ * (the same workspace size; the same results). */
+int tbvh_knn_accel_routed_tail(const void* true_accel, const float* true_node_aabbs,
+                               int64_t true_num_real_nodes, const void* false_accel,
+                               const float* false_node_aabbs, int64_t false_num_real_nodes,
+                               const float* queries, const uint8_t* routes, const int64_t* order,
+                               int64_t B, int64_t M, int64_t true_num_leaves,
+                               int64_t false_num_leaves, int D, int k,
+                               int64_t* out_indices, float* out_distances,
+                               void* workspace, size_t workspace_bytes, void* stream);
+
 /* Cell-block form of tbvh_knn_accel_routed_spatial, for the same binding
  * (no counterpart in the reference; identical results): each query first
  * searches the block of grid cells around it in its route's structure (as

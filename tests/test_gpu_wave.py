@@ -97,3 +97,86 @@ def test_wave_search_non_finite(monkeypatch):
     wave, plain = _both(monkeypatch, lambda: tb.query_knn(bvh, tq, 8))
     for a, b in zip(wave, plain):
         assert torch.equal(a, b)
+
+
+# Queries near a shell's centre are nearly equidistant from all of it, so the
+# traversal's waves pass their budget of iterations and give them up
+# (tbvh_knn_*_tail); the wave search of the same call is the reference.
+def _shell(n, dim, seed):
+    g = torch.Generator("cuda").manual_seed(seed)
+    v = torch.randn((n, dim), generator=g, device="cuda")
+    return v / v.norm(dim=1, keepdim=True) * (1.0 + 1e-3 * torch.rand((n, 1), generator=g, device="cuda"))
+
+
+def _centre(m, dim, seed):
+    g = torch.Generator("cuda").manual_seed(seed)
+    return 0.3 * torch.randn((m, dim), generator=g, device="cuda")
+
+
+@pytest.mark.parametrize("dim,k", [(2, 4), (2, 32), (3, 8), (3, 16), (3, 32)])
+@pytest.mark.parametrize("layout", ["batched", "rows", "ordered", "ragged", "grid"])
+def test_given_up_queries(monkeypatch, layout, dim, k):
+    pts = torch.stack([_shell(33_000, dim, s) for s in (1, 2)])
+    m = 70_000 if layout == "grid" else 15_000  # more than 2^17 queries: the cell-block search's fallback
+    q = torch.stack([_centre(m, dim, s) for s in (3, 4)])
+    if layout == "ragged":
+        off = torch.tensor([0, 33_000, 66_000 - 7], device="cuda")
+        qoff = torch.tensor([0, 15_000 + 3, 30_000], device="cuda")
+        bvh = tb.build_bvh(pts.reshape(-1, dim)[:-7].contiguous(), batch_offsets=off)
+        call = lambda: tb.query_knn(bvh, q.reshape(-1, dim), k, query_offsets=qoff)  # noqa: E731
+    else:
+        d = _C.build_bvh_batched_cooperative(pts)
+        args = (d["node_aabbs"], d["sorted_indices"], q)
+        tail = (d["num_leaves"], d["num_real_nodes"], dim, k)
+        order = _C.morton_sort_queries_narrow(q, d["scene_min"], d["scene_max"])
+        if layout == "ordered":
+            call = lambda: _C.query_knn_batched_cached_bounds_ordered(*args, order, *tail)  # noqa: E731
+        else:
+            src = pts if layout == "rows" else None
+            call = lambda: _C.query_knn_batched_cached_bounds(*args, *tail, source_points=src)  # noqa: E731
+    wave, plain = _both(monkeypatch, call)
+    for a, b in zip(wave, plain):
+        assert torch.equal(a, b)
+    if layout == "batched":
+        rows = torch.arange(0, m, 997, device="cuda")
+        ei, ed = oracle.knn(pts[1].cpu().numpy(), q[1, rows].cpu().numpy(), k)
+        assert np.array_equal(plain[0][1, rows].cpu().numpy(), ei)
+        assert np.array_equal(plain[1][1, rows].cpu().numpy().view(np.uint32), ed.view(np.uint32))
+
+
+def test_queries_are_given_up():
+    """The tail entry point marks queries here, and its rows are the plain
+    traversal's."""
+    L = _native.load()
+    pts, q = _shell(33_000, 3, 1)[None], _centre(30_000, 3, 3)[None]
+    d = _C.build_bvh_batched_cooperative(pts, with_accel=True)
+    ws = torch.zeros(_native._size(L.tbvh_knn_tail_workspace_size, 30_000, 3), dtype=torch.uint8, device="cuda")
+    out = [(torch.empty((30_000, 16), dtype=torch.int64, device="cuda"),
+            torch.empty((30_000, 16), dtype=torch.float32, device="cuda")) for _ in range(2)]
+    p, stream = _native._ptr, _native._stream(pts.device)
+    _native._check(L.tbvh_knn_accel_tail(p(d["accel"]), p(d["node_aabbs"]), d["num_real_nodes"], p(q), None, 1, 30_000,
+                                         33_000, 3, 16, 0, None, 0, p(out[0][0]), p(out[0][1]), None, p(ws),
+                                         ws.numel(), stream))
+    _native._check(L.tbvh_knn_accel(p(d["accel"]), p(q), None, 1, 30_000, 33_000, 3, 16, p(out[1][0]), p(out[1][1]),
+                                    stream))
+    masks = ws[: (30_000 + 63) // 64 * 8].view(torch.int64)
+    assert int((masks != 0).sum()) > 100
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("dim,k", [(2, 8), (3, 16)])
+def test_given_up_routed_queries(dim, k):
+    a, b = _shell(20_000, dim, 1)[None], 1.5 * _shell(9_000, dim, 2)[None]
+    q = _centre(30_000, dim, 3)[None]
+    routes = torch.arange(30_000, device="cuda")[None] % 3 == 0
+    t, f = _C.build_bvh_batched_cooperative(a), _C.build_bvh_batched_cooperative(b)
+    order = torch.arange(30_000, device="cuda")[None].contiguous()
+    i, d2 = _C.query_knn_routed_batched_cached_bounds_spatial(
+        t["node_aabbs"], t["sorted_indices"], f["node_aabbs"], f["sorted_indices"], q, routes, order,
+        t["num_leaves"], t["num_real_nodes"], f["num_leaves"], f["num_real_nodes"], dim, k)
+    for payload, sel, offset in ((t, routes[0], 0), (f, ~routes[0], 20_000)):
+        qs = q[:, sel].contiguous()
+        ei, ed = _C.query_knn_batched_cached_bounds(payload["node_aabbs"], payload["sorted_indices"], qs,
+                                                    payload["num_leaves"], payload["num_real_nodes"], dim, k)
+        assert torch.equal(i[0, sel], ei[0] + offset)
+        assert torch.equal(d2[0, sel], ed[0])

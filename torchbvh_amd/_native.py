@@ -122,6 +122,22 @@ def _declare(L) -> None:
     L.tbvh_knn_accel_wave.argtypes = (
         [_vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _int, _int, _int, _vp, _int, _vp, _vp, _vp, _vp]
     )
+    L.tbvh_knn_accel_ragged_wave.argtypes = (
+        [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _int, _int, _vp, _int, _vp, _vp, _vp, _vp]
+    )
+    L.tbvh_knn_accel_routed_tail.argtypes = (
+        [_vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp, _vp, _vp,
+         ctypes.c_size_t, _vp]
+    )
+    L.tbvh_knn_tail_workspace_size.argtypes = [_i64, _int, _vp]
+    L.tbvh_knn_accel_tail.argtypes = (
+        [_vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _int, _int, _int, _vp, _int, _vp, _vp, _vp, _vp,
+         ctypes.c_size_t, _vp]
+    )
+    L.tbvh_knn_accel_ragged_tail.argtypes = (
+        [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _int, _int, _vp, _int, _vp, _vp, _vp, _vp,
+         ctypes.c_size_t, _vp]
+    )
     L.tbvh_knn_accel_ragged_positions.argtypes = (
         [_vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _int, _int, _vp, _int, _vp, _vp, _vp, _vp]
     )
@@ -137,6 +153,7 @@ def _declare(L) -> None:
         "tbvh_knn_accel", "tbvh_knn_accel_ragged", "tbvh_knn_spatial", "tbvh_knn_accel_spatial",
         "tbvh_knn_accel_grid_workspace_size", "tbvh_knn_accel_grid", "tbvh_knn_accel_grid_spatial",
         "tbvh_knn_accel_positions", "tbvh_knn_accel_grid_positions", "tbvh_knn_accel_ragged_positions", "tbvh_knn_accel_wave",
+        "tbvh_knn_accel_ragged_wave", "tbvh_knn_accel_routed_tail", "tbvh_knn_tail_workspace_size", "tbvh_knn_accel_tail", "tbvh_knn_accel_ragged_tail",
         "tbvh_sort_routed_queries_workspace_size", "tbvh_sort_routed_queries",
         "tbvh_knn_routed_spatial", "tbvh_knn_accel_routed_spatial",
         "tbvh_knn_accel_routed_grid_workspace_size", "tbvh_knn_accel_routed_grid_spatial",
@@ -241,20 +258,18 @@ MAX_ACCEL_CLOUD = 1 << 28
 # than it saves.
 GRID_MIN_QUERIES = 1 << 17
 
-# Batched accel k-NN calls of at most this many queries search with one wave
-# per query (tbvh_knn_accel_wave); the traversal takes one query per lane and
-# its time hardly depends on the number of queries until they fill the chip.
-# Measured (call, wave / traversal, us).  3-D, uniform: 50,000 points, 1,000
-# queries k = 8 23 / 73; 10,000 points, 8,000 queries k = 4 29 / 58; 300,000
-# points, 16,000 queries k = 4 98 / 97, k = 16 129 / 147, 32,000 queries k = 16
-# 210 / 151; clustered or surface clouds with queries away from the points gain
-# most (50,000 on a surface, 16,000 queries k = 16 119 / 913).  2-D boxes
-# overlap less, so the traversal is shorter: 10,000 points, 8,000 queries k =
-# 4 23 / 31, 16,000 34 / 32; 300,000 points, 4,000 queries k = 4 40 / 41, 8,000
-# 59 / 40.
-WAVE_MAX_QUERIES = 1 << 14          # 3-D
-WAVE_MAX_QUERIES_2D = 1 << 13       # 2-D, clouds of at most WAVE_2D_CLOUD points
-WAVE_MAX_QUERIES_2D_LARGE = 1 << 12
+# Accel k-NN calls of at most this many queries search with one wave per query
+# (tbvh_knn_accel_wave); the traversal takes one query per lane and its time
+# hardly depends on the number of queries until they fill the chip.  Measured
+# (call, wave / traversal, us).  3-D, uniform: 50,000 points, 1,000 queries k = 8
+# 24 / 76, 32,000 queries k = 4 83 / 72, k = 8 94 / 94; 300,000 points, 16,000
+# queries k = 4 90 / 104, 32,000 137 / 119.  2-D boxes overlap less, so the
+# traversal is shorter: 10,000 points, 16,000 queries k = 4 32 / 34; 50,000 points,
+# 8,000 queries k = 4 30 / 39, 16,000 45 / 39; 300,000 points, 4,000 queries k = 4
+# 40 / 44, 8,000 57 / 43, k = 8 57 / 64.
+WAVE_MAX_QUERIES = 24 << 10         # 3-D
+WAVE_MAX_QUERIES_2D = 12 << 10      # 2-D, clouds of at most WAVE_2D_CLOUD points
+WAVE_MAX_QUERIES_2D_LARGE = 6 << 10
 WAVE_2D_CLOUD = 1 << 16
 
 
@@ -843,12 +858,7 @@ class _NativeOps:
                     _ptr(accel), _ptr(node_aabbs), int(num_real_nodes), _ptr(query_points), _ptr(query_order),
                     B, M, int(num_leaves), int(dim), int(k), _ptr(source_points), C, _ptr(indices),
                     _ptr(distances), _ptr(positions), _ptr(ws), need, _stream(dev)))
-            elif fused:
-                _check(L.tbvh_knn_accel_positions(
-                    _ptr(accel), _ptr(query_points), _ptr(query_order), B, M, int(num_leaves),
-                    int(dim), int(k), _ptr(source_points), C, _ptr(indices), _ptr(distances),
-                    _ptr(positions), _stream(dev)))
-            elif grid:
+            elif grid and not fused:
                 need = _grid_workspace_size(B, M, int(num_leaves), int(dim), int(k))
                 # The cell-block search first (same results; see
                 # tbvh_knn_accel_grid), where the clouds allow a grid and
@@ -860,10 +870,12 @@ class _NativeOps:
                     B, M, int(num_leaves), int(dim), int(k), _ptr(indices), _ptr(distances),
                     _ptr(ws), need, _stream(dev)))
             elif accel is not None:
-                fn = L.tbvh_knn_accel_spatial if spatial else L.tbvh_knn_accel
-                _check(fn(
-                    _ptr(accel), _ptr(query_points), _ptr(query_order), B, M, int(num_leaves),
-                    int(dim), int(k), _ptr(indices), _ptr(distances), _stream(dev)))
+                ws = _workspace(_size(L.tbvh_knn_tail_workspace_size, B * M, int(dim)), dev)
+                _check(L.tbvh_knn_accel_tail(
+                    _ptr(accel), _ptr(node_aabbs), int(num_real_nodes), _ptr(query_points), _ptr(query_order),
+                    B, M, int(num_leaves), int(dim), int(k), int(spatial), _ptr(source_points) if fused else None,
+                    C if fused else 0, _ptr(indices), _ptr(distances), _ptr(positions), _ptr(ws), ws.numel(),
+                    _stream(dev)))
             else:
                 fn = L.tbvh_knn_spatial if spatial else L.tbvh_knn
                 _check(fn(
@@ -998,10 +1010,12 @@ class _NativeOps:
                     _ptr(query_order), B, M, int(true_num_leaves), int(false_num_leaves), int(dim), int(k),
                     _ptr(indices), _ptr(distances), _ptr(ws), need, _stream(dev)))
             elif true_accel is not None and false_accel is not None:
-                _check(L.tbvh_knn_accel_routed_spatial(
-                    _ptr(true_accel), _ptr(false_accel), _ptr(query_points), _ptr(routes),
-                    _ptr(query_order), B, M, int(true_num_leaves), int(false_num_leaves), int(dim),
-                    int(k), _ptr(indices), _ptr(distances), _stream(dev)))
+                ws = _workspace(_size(L.tbvh_knn_tail_workspace_size, B * M, int(dim)), dev)
+                _check(L.tbvh_knn_accel_routed_tail(
+                    _ptr(true_accel), _ptr(true_node_aabbs), int(true_num_real_nodes), _ptr(false_accel),
+                    _ptr(false_node_aabbs), int(false_num_real_nodes), _ptr(query_points), _ptr(routes),
+                    _ptr(query_order), B, M, int(true_num_leaves), int(false_num_leaves), int(dim), int(k),
+                    _ptr(indices), _ptr(distances), _ptr(ws), ws.numel(), _stream(dev)))
             else:
                 _check(L.tbvh_knn_routed_spatial(
                     _ptr(true_node_aabbs), _ptr(true_sorted_indices), _ptr(false_node_aabbs),
@@ -1045,16 +1059,19 @@ class _NativeOps:
             return indices, distances, source_points.new_empty((0, k) + tuple(source_points.shape[1:]))
         L = load()
         with torch.cuda.device(dev):
-            if fused:
-                _check(L.tbvh_knn_accel_ragged_positions(
-                    _ptr(accel), _ptr(point_offsets), int(total_points), _ptr(query_points),
-                    _ptr(query_offsets), _ptr(query_order), int(batch_size), T, int(dim), int(k),
-                    _ptr(source_points), C, _ptr(indices), _ptr(distances), _ptr(positions), _stream(dev)))
+            if accel is not None and T <= _wave_limit(int(dim), int(total_points)):
+                _check(L.tbvh_knn_accel_ragged_wave(
+                    _ptr(accel), _ptr(node_aabbs), _ptr(node_offsets), _ptr(point_offsets), int(total_points),
+                    _ptr(query_points), _ptr(query_offsets), _ptr(query_order), int(batch_size), T, int(dim), int(k),
+                    _ptr(source_points) if fused else None, C if fused else 0, _ptr(indices), _ptr(distances),
+                    _ptr(positions), _stream(dev)))
             elif accel is not None:
-                _check(L.tbvh_knn_accel_ragged(
-                    _ptr(accel), _ptr(point_offsets), int(total_points), _ptr(query_points),
-                    _ptr(query_offsets), _ptr(query_order), int(batch_size), T, int(dim), int(k),
-                    _ptr(indices), _ptr(distances), _stream(dev)))
+                ws = _workspace(_size(L.tbvh_knn_tail_workspace_size, T, int(dim)), dev)
+                _check(L.tbvh_knn_accel_ragged_tail(
+                    _ptr(accel), _ptr(node_aabbs), _ptr(node_offsets), _ptr(point_offsets), int(total_points),
+                    _ptr(query_points), _ptr(query_offsets), _ptr(query_order), int(batch_size), T, int(dim), int(k),
+                    _ptr(source_points) if fused else None, C if fused else 0, _ptr(indices), _ptr(distances),
+                    _ptr(positions), _ptr(ws), ws.numel(), _stream(dev)))
             else:
                 _check(L.tbvh_knn_ragged(
                     _ptr(node_aabbs), _ptr(sorted_indices), _ptr(point_offsets), _ptr(node_offsets),

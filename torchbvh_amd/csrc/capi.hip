@@ -955,7 +955,7 @@ static int knn_accel_batched(const char* op, const void* accel, const float* que
                              void* stream_ptr, const float* source_points = nullptr, int source_cols = 0,
                              float* out_positions = nullptr, const float* node_aabbs = nullptr,
                              int64_t num_real_nodes = 0, void* ws = nullptr, size_t ws_bytes = 0,
-                             bool wave = false) {
+                             bool wave = false, bool tail = false) {
     if (int r = check_dim(op, D)) return r;
     if (!supported_k(k)) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: k must be 4, 8, or 16 (32 is also supported), got %d", op, k);
     if (B < 1 || M < 0) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: need B >= 1 and M >= 0", op);
@@ -985,8 +985,8 @@ static int knn_accel_batched(const char* op, const void* accel, const float* que
     a.source_points = source_points;
     a.source_cols = source_cols;
     a.out_positions = out_positions;
-    const int level = ws ? grid_level(num_leaves, D, k) : 0;
-    if (level > 0 || wave) {
+    const int level = ws && !tail ? grid_level(num_leaves, D, k) : 0;
+    if (level > 0 || wave || tail) {
         if (!node_aabbs) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: null node_aabbs", op);
         if (num_real_nodes != tree::real_node_count(static_cast<int>(num_leaves))) {
             return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: num_real_nodes does not match num_leaves", op);
@@ -995,7 +995,16 @@ static int knn_accel_batched(const char* op, const void* accel, const float* que
     if (wave) {
         a.node_aabbs = node_aabbs;
         a.num_real_nodes = static_cast<int32_t>(num_real_nodes);
-        TBVH_TRY(op, launch_knn_wave(a, D, k, static_cast<hipStream_t>(stream_ptr)));
+        TBVH_TRY(op, launch_knn_wave(a, D, k, false, static_cast<hipStream_t>(stream_ptr)));
+        return ok();
+    }
+    if (tail && tail_workspace_bytes(B * M, D) > 0) {
+        if (int r = check_workspace(op, ws, ws_bytes, tail_workspace_bytes(B * M, D))) return r;
+        a.node_aabbs = node_aabbs;
+        a.num_real_nodes = static_cast<int32_t>(num_real_nodes);
+        set_tail(a, ws);
+        TBVH_TRY(op, launch_knn_accel(a, D, k, false, static_cast<hipStream_t>(stream_ptr)));
+        TBVH_TRY(op, launch_knn_tail(a, D, k, false, static_cast<hipStream_t>(stream_ptr)));
         return ok();
     }
     if (level > 0) {
@@ -1062,7 +1071,9 @@ static int knn_accel_ragged(const char* op, const void* accel, const int64_t* po
                             int64_t total_points, const float* queries, const int64_t* query_offsets,
                             const int64_t* order, int64_t B, int64_t total_q, int D, int k,
                             int64_t* out_indices, float* out_distances, void* stream_ptr,
-                            const float* source_points, int source_cols, float* out_positions) {
+                            const float* source_points, int source_cols, float* out_positions,
+                            const float* node_aabbs = nullptr, const int64_t* node_offsets = nullptr,
+                            void* ws = nullptr, size_t ws_bytes = 0, bool tail = false, bool wave = false) {
     if (int r = check_dim(op, D)) return r;
     if (!supported_k(k)) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: k must be 4, 8, or 16 (32 is also supported), got %d", op, k);
     if (B < 1 || total_q < 0) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: need B >= 1 and total_q >= 0", op);
@@ -1088,7 +1099,24 @@ static int knn_accel_ragged(const char* op, const void* accel, const int64_t* po
     a.source_points = source_points;
     a.source_cols = source_cols;
     a.out_positions = out_positions;
+    if (tail || wave) {
+        if (!node_aabbs || !node_offsets) {
+            return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: null node_aabbs or node_offsets", op);
+        }
+        a.node_aabbs = node_aabbs;
+        a.node_offsets = node_offsets;
+    }
+    if (wave) {
+        TBVH_TRY(op, launch_knn_wave(a, D, k, true, static_cast<hipStream_t>(stream_ptr)));
+        return ok();
+    }
+    tail = tail && tail_workspace_bytes(total_q, D) > 0;
+    if (tail) {
+        if (int r = check_workspace(op, ws, ws_bytes, tail_workspace_bytes(total_q, D))) return r;
+        set_tail(a, ws);
+    }
     TBVH_TRY(op, launch_knn_accel(a, D, k, true, static_cast<hipStream_t>(stream_ptr)));
+    if (tail) TBVH_TRY(op, launch_knn_tail(a, D, k, true, static_cast<hipStream_t>(stream_ptr)));
     return ok();
 }
 
@@ -1142,6 +1170,59 @@ int tbvh_knn_accel_wave(const void* accel, const float* node_aabbs, int64_t num_
     return knn_accel_batched(op, accel, queries, order, B, M, num_leaves, D, k, spatial != 0, out_indices,
                              out_distances, stream_ptr, source_points, source_cols, out_positions, node_aabbs,
                              num_real_nodes, nullptr, 0, true);
+}
+
+int tbvh_knn_tail_workspace_size(int64_t total_q, int D, size_t* bytes) {
+    const char* op = "tbvh_knn_tail_workspace_size";
+    if (!bytes) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: null output pointer", op);
+    if (total_q < 0 || total_q > kMaxRows) {
+        return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: total query count must fit in signed int32", op);
+    }
+    if (int r = check_dim(op, D)) return r;
+    *bytes = tail_workspace_bytes(total_q, D);
+    return ok();
+}
+
+int tbvh_knn_accel_tail(const void* accel, const float* node_aabbs, int64_t num_real_nodes, const float* queries,
+                        const int64_t* order, int64_t B, int64_t M, int64_t num_leaves, int D, int k, int spatial,
+                        const float* source_points, int source_cols, int64_t* out_indices, float* out_distances,
+                        float* out_positions, void* ws, size_t ws_bytes, void* stream_ptr) {
+    const char* op = "tbvh_knn_accel_tail";
+    if (source_points || out_positions) {
+        if (int r = check_positions(op, source_points, source_cols, out_positions)) return r;
+    }
+    return knn_accel_batched(op, accel, queries, order, B, M, num_leaves, D, k, spatial != 0, out_indices,
+                             out_distances, stream_ptr, source_points, source_cols, out_positions, node_aabbs,
+                             num_real_nodes, ws, ws_bytes, false, true);
+}
+
+int tbvh_knn_accel_ragged_tail(const void* accel, const float* node_aabbs, const int64_t* node_offsets,
+                               const int64_t* point_offsets, int64_t total_points, const float* queries,
+                               const int64_t* query_offsets, const int64_t* order, int64_t B, int64_t total_q, int D,
+                               int k, const float* source_points, int source_cols, int64_t* out_indices,
+                               float* out_distances, float* out_positions, void* ws, size_t ws_bytes,
+                               void* stream_ptr) {
+    const char* op = "tbvh_knn_accel_ragged_tail";
+    if (source_points || out_positions) {
+        if (int r = check_positions(op, source_points, source_cols, out_positions)) return r;
+    }
+    return knn_accel_ragged(op, accel, point_offsets, total_points, queries, query_offsets, order, B, total_q, D, k,
+                            out_indices, out_distances, stream_ptr, source_points, source_cols, out_positions,
+                            node_aabbs, node_offsets, ws, ws_bytes, true);
+}
+
+int tbvh_knn_accel_ragged_wave(const void* accel, const float* node_aabbs, const int64_t* node_offsets,
+                               const int64_t* point_offsets, int64_t total_points, const float* queries,
+                               const int64_t* query_offsets, const int64_t* order, int64_t B, int64_t total_q, int D,
+                               int k, const float* source_points, int source_cols, int64_t* out_indices,
+                               float* out_distances, float* out_positions, void* stream_ptr) {
+    const char* op = "tbvh_knn_accel_ragged_wave";
+    if (source_points || out_positions) {
+        if (int r = check_positions(op, source_points, source_cols, out_positions)) return r;
+    }
+    return knn_accel_ragged(op, accel, point_offsets, total_points, queries, query_offsets, order, B, total_q, D, k,
+                            out_indices, out_distances, stream_ptr, source_points, source_cols, out_positions,
+                            node_aabbs, node_offsets, nullptr, 0, false, true);
 }
 
 int tbvh_knn_accel_ragged_positions(const void* accel, const int64_t* point_offsets, int64_t total_points,
@@ -1306,6 +1387,39 @@ int tbvh_knn_accel_routed_grid_spatial(const void* true_accel, const float* true
         return ok();
     }
     TBVH_TRY(op, launch_knn_accel(a, D, k, false, stream));
+    return ok();
+}
+
+int tbvh_knn_accel_routed_tail(const void* true_accel, const float* true_node_aabbs, int64_t true_num_real_nodes,
+                               const void* false_accel, const float* false_node_aabbs, int64_t false_num_real_nodes,
+                               const float* queries, const uint8_t* routes, const int64_t* order, int64_t B,
+                               int64_t M, int64_t true_num_leaves, int64_t false_num_leaves, int D, int k,
+                               int64_t* out_indices, float* out_distances, void* ws, size_t ws_bytes,
+                               void* stream_ptr) {
+    const char* op = "tbvh_knn_accel_routed_tail";
+    KnnArgs a{};
+    if (int r = routed_accel_args(op, true_accel, false_accel, queries, routes, order, B, M, true_num_leaves,
+                                  false_num_leaves, D, k, out_indices, out_distances, a)) {
+        return r;
+    }
+    if (M == 0) return ok();
+    if (!true_node_aabbs || !false_node_aabbs) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: null node_aabbs", op);
+    if (true_num_real_nodes != tree::real_node_count(static_cast<int>(true_num_leaves)) ||
+        false_num_real_nodes != tree::real_node_count(static_cast<int>(false_num_leaves))) {
+        return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: num_real_nodes does not match num_leaves", op);
+    }
+    const bool tail = tail_workspace_bytes(B * M, D) > 0;
+    if (tail) {
+        if (int r = check_workspace(op, ws, ws_bytes, tail_workspace_bytes(B * M, D))) return r;
+        set_tail(a, ws);
+    }
+    a.node_aabbs = true_node_aabbs;
+    a.num_real_nodes = static_cast<int32_t>(true_num_real_nodes);
+    a.node_aabbs2 = false_node_aabbs;
+    a.num_real_nodes2 = static_cast<int32_t>(false_num_real_nodes);
+    const hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
+    TBVH_TRY(op, launch_knn_accel(a, D, k, false, stream));
+    if (tail) TBVH_TRY(op, launch_knn_tail(a, D, k, false, stream));
     return ok();
 }
 

@@ -231,32 +231,6 @@ __device__ __forceinline__ void merge_candidates12(uint64_t (&best)[K], uint64_t
     }
 }
 
-// One wave per work-group: measured against 256 threads, -3.5% at cfg2 and
-// -14% at cfg5, whose waves differ most in cost (finer-grained balancing
-// over the CUs); 128 falls between, 512 is 13-24% slower.
-constexpr int kKnnBlock = 64;
-constexpr int kXcds = 8;               // MI355X: work-groups are dealt round-robin over 8 XCDs
-
-// The cell-block search's failure lists (launch positions left for the next
-// stage) are cut into kXcds * kGridSubLists sub-lists, each with its own
-// count, filled by one atomic add per wave.  Work-group b's sub-list is that
-// of its XCD share (b % kXcds, as in the tile map) and of the residue of its
-// local tile index (b / kXcds) mod kGridSubLists; the next stage's
-// work-group b reads chunk (b / kXcds) / kGridSubLists of the same
-// sub-list, so that it takes failures of tiles near its own.  One count per
-// XCD share measured 375 us for the first pass at cfg3, where every wave
-// fails at once: same-address atomics serialise (about 90 ns each).  The
-// counts lie kCountStride words apart, each on a 128-byte line of its own.
-constexpr int kGridSubLists = 64;
-constexpr int kCountStride = 32;
-constexpr int kGridCounts = kXcds * kGridSubLists;  // per list
-__device__ __forceinline__ int grid_sublist() {
-    return static_cast<int>(blockIdx.x % kXcds) * kGridSubLists + static_cast<int>(blockIdx.x / kXcds) % kGridSubLists;
-}
-__device__ __forceinline__ int64_t grid_chunk_start() {
-    return static_cast<int64_t>(blockIdx.x / kXcds / kGridSubLists) * kKnnBlock;
-}
-
 // Entries of a lane's deferred-node stack, all in LDS (6 bytes each: a
 // 32-bit child ref and a 16-bit distance, in columns of stride kKnnBlock):
 // as many as the LDS budget of each (D, k) holds.  7.5 KB per work-group for
@@ -653,6 +627,13 @@ struct HeapNodes {
 // 12 candidates instead of 168; cfg5 traversal 22.5 -> 20.4 ms (both at 3
 // waves per SIMD).  At k = 16 two slots measured +1.5-2% (cfg2, cfg3).
 //
+// Budget.  A wave that has flushed `budget` times gives up the queries it
+// has not finished: they end with lost_min = -1 and are searched again by one
+// wave each (launch_knn_tail), from the k-th distance reached.  A query far
+// from a surface or a cluster, nearly as far from thousands of its points,
+// otherwise holds its wave, and the call, for up to a millisecond.  (Counted
+// per loop iteration instead of per flush: +2 to 3% on every traversal.)
+//
 // Without kPostpone, buckets are scanned when reached, so the traversal makes
 // the reference's visits in the reference's order.  The implicit tree runs
 // that way: where the result does depend on the order (points with a NaN
@@ -660,7 +641,7 @@ struct HeapNodes {
 // reference's result.
 template <bool kPostpone, int K, int L, bool kCompact, class Nodes>
 __device__ __forceinline__ void traverse(const Nodes& t, const float* q, uint64_t (&best)[K],
-                                         RingStack<L, kCompact>& stack) {
+                                         RingStack<L, kCompact>& stack, int budget) {
     // 3-D k = 32 parks two buckets per lane and merges them together.
     constexpr bool kTwoSlots = kPostpone && K >= 32 && Nodes::kDims == 3;
     int32_t ref = t.root();
@@ -669,6 +650,7 @@ __device__ __forceinline__ void traverse(const Nodes& t, const float* q, uint64_
     int32_t parked2 = Nodes::kNone;
     bool waiting = false;
     bool done = false;
+    int steps = 0;
 
     // Wave priority: between flushes a wave runs a chain of dependent record
     // loads (visit, push, pop), and its next load should issue as soon as
@@ -706,6 +688,10 @@ __device__ __forceinline__ void traverse(const Nodes& t, const float* q, uint64_
                 parked = Nodes::kNone;
                 parked2 = Nodes::kNone;
                 waiting = false;
+                if (++steps == budget && !done) {
+                    done = true;
+                    stack.lost_min = -1.0f;
+                }
                 __builtin_amdgcn_s_setprio(1);
             }
         }
@@ -789,56 +775,6 @@ __device__ __forceinline__ void traverse(const Nodes& t, const float* q, uint64_
 // own L2; logical tile t = (block % 8) * (grid / 8) + block / 8 gives every
 // XCD a contiguous run of Morton-ordered queries, so one XCD's L2 serves a
 // compact region of the tree.
-// Where query `gid` of the launch reads and writes: its cloud, its input row
-// and output row, and the structure it searches.
-struct QueryLoc {
-    int64_t row;           // input row (queries), -1 for a corrupt order entry
-    int64_t out_row;       // result row
-    int64_t pstart;        // the cloud's first point row
-    int64_t nstart;        // the cloud's first node row (implicit tree)
-    int64_t index_offset;  // added to result indices (false route)
-    int n;                 // the cloud's points
-    bool second;           // false route: the second structure
-};
-
-template <bool kOrdered, bool kRagged, bool kRouted, bool kAccel>
-__device__ __forceinline__ QueryLoc locate(const KnnArgs& a, int64_t gid) {
-    QueryLoc l;
-    int64_t seg, qbase, qcount;
-    if constexpr (kRagged) {
-        seg = find_segment([&](int i) { return a.query_offsets[i]; }, static_cast<int>(a.B), gid);
-        qbase = a.query_offsets[seg];
-        qcount = a.query_offsets[seg + 1] - qbase;
-        l.pstart = a.point_offsets[seg];
-        l.n = static_cast<int>(a.point_offsets[seg + 1] - l.pstart);
-        l.nstart = kAccel ? 0 : a.node_offsets[seg];
-    } else {
-        seg = gid / a.M;
-        qbase = seg * a.M;
-        qcount = a.M;
-        l.n = a.num_leaves;
-        l.pstart = seg * static_cast<int64_t>(l.n);
-        l.nstart = seg * static_cast<int64_t>(a.num_real_nodes);
-    }
-    const int64_t local = gid - qbase;
-    const int64_t qi = kOrdered ? a.order[qbase + local] : local;
-    l.row = qi < 0 || qi >= qcount ? -1 : qbase + qi;  // a corrupt order never indexes out of range
-    // Spatial output (knn_query.cu:147-148) keeps the launch (Morton) order.
-    l.out_row = a.spatial_output ? gid : l.row;
-    l.second = false;
-    l.index_offset = 0;
-    if (kRouted && l.row >= 0 && a.routes[l.row] == 0) {
-        // False route (knn_query.cu:205-217): the second structure, indices
-        // after the first's points.
-        l.second = true;
-        l.index_offset = l.n;
-        l.n = a.num_leaves2;
-        l.pstart = seg * static_cast<int64_t>(l.n);
-        l.nstart = seg * static_cast<int64_t>(a.num_real_nodes2);
-    }
-    return l;
-}
-
 template <int D, int K, bool kOrdered, bool kRagged, bool kRouted, bool kAccel, bool kCompact>
 __device__ __forceinline__ void knn_query(const KnnArgs& a) {
     constexpr int kLds = lds_stack_entries<D, K>();
@@ -859,12 +795,20 @@ __device__ __forceinline__ void knn_query(const KnnArgs& a) {
     if (fallback) {
         const int64_t listed = a.fb_count[grid_sublist() * kCountStride];
         const int64_t at = grid_chunk_start() + threadIdx.x;
-        if (at >= listed) return;
-        gid = a.fb_list[grid_sublist() * a.fb_seg + at];
-        seed = a.fb_bound[gid];
+        gid = a.total_q;
+        if (at < listed) {
+            gid = a.fb_list[grid_sublist() * a.fb_seg + at];
+            seed = a.fb_bound[gid];
+        }
     }
-    if (gid >= a.total_q) return;
-    const QueryLoc in = locate<kOrdered, kRagged, kRouted, kAccel>(a, gid);
+    QueryLoc in{};
+    in.row = -1;
+    if (gid < a.total_q) in = locate<kOrdered, kRagged, kRouted, kAccel>(a, gid);
+    const bool tail = kAccel && a.tail_masks != nullptr;
+    if (__ballot(in.row >= 0) == 0) {
+        if (tail && threadIdx.x == 0) a.tail_masks[blockIdx.x] = 0;
+        return;
+    }
     if (in.row < 0) return;
 
     float q[D];
@@ -891,12 +835,12 @@ __device__ __forceinline__ void knn_query(const KnnArgs& a) {
         t.recs = kRows ? recs : recs + in.pstart * AccelNodes<D, kRows>::R;
         t.first_row = kRows ? static_cast<int>(in.pstart) : 0;
         t.n = in.n;
-        traverse<true>(t, q, best, stack);
+        traverse<true>(t, q, best, stack, tail ? a.tail_budget : INT32_MAX);
     } else {
         HeapNodes<D> t;
         t.init((in.second ? a.node_aabbs2 : a.node_aabbs) + in.nstart * 2 * D,
                (in.second ? a.sorted_indices2 : a.sorted_indices) + in.pstart, in.n);
-        traverse<false>(t, q, best, stack);
+        traverse<false>(t, q, best, stack, INT32_MAX);
     }
 
     // The output location is derived again from the lane's position (the
@@ -905,6 +849,17 @@ __device__ __forceinline__ void knn_query(const KnnArgs& a) {
     // two apart, so nothing of the first derivation stays live.
     int64_t gid_out = tile * kKnnBlock + __lane_id();
     if (fallback) gid_out = a.fb_list[grid_sublist() * a.fb_seg + grid_chunk_start() + __lane_id()];
+    if (tail) {
+        // Only the lanes still here vote; bits of the others stay clear.
+        const bool given_up = stack.lost_min < 0.0f;
+        const uint64_t left = __ballot(given_up);
+        const int leader = __ffsll(static_cast<long long>(__ballot(1))) - 1;
+        if (lane_id() == leader) a.tail_masks[blockIdx.x] = left;
+        if (given_up) {
+            a.tail_bounds[gid_out] = __uint_as_float(static_cast<uint32_t>(best[K - 1] >> 32));
+            return;
+        }
+    }
     const QueryLoc out = locate<kOrdered, kRagged, kRouted, kAccel>(a, gid_out);
     write_results<K, D>(a, out.out_row, best, out.index_offset, out.pstart);
 }
@@ -1752,6 +1707,42 @@ int grid_level(int64_t n, int D, int K) {
 }
 
 namespace {
+int64_t traversal_groups(int64_t total_q) {
+    const int64_t tiles = (total_q + kKnnBlock - 1) / kKnnBlock;
+    return (tiles + kXcds - 1) / kXcds * kXcds;
+}
+// Flushes of a traversal wave before it gives up its unfinished queries.  A
+// wave on uniform points ends within about 40 (3-D, k = 16 and 32: a budget
+// of 32 measured +40%, 48 nothing).  With few waves the call lasts as long
+// as its slowest one and the chip idles meanwhile, so that one is cut early;
+// with more waves than fit at once a query given up costs more than the lane
+// slots it frees, unless its search is long.  Measured, call in us without a
+// budget / 48 / 96 / 128 / 256: 50,000 surface points and box queries, k = 16
+// 1251 / 648 / 599 / 688 / 1001; 200,003 surface points, self-queries 308 / 233 /
+// 310 / 309 / 311; 100,000 and 400,000 queries 2611 / 1448 / 1358 / 1259 / 1758;
+// 300,000 and 1M 4733 / 5456 / 4432 / 4026 / 3510; 6M queries of 64 surface
+// clouds, k = 32 16113 / 28811 / 21285 / 18026 / 15337.
+int tail_budget(int64_t total_q) {
+    return static_cast<int>(std::min<int64_t>(std::max<int64_t>(16 + traversal_groups(total_q) / 64, 56), 256));
+}
+size_t tail_masks_bytes(int64_t total_q) { return (static_cast<size_t>(traversal_groups(total_q)) * 8 + 255) / 256 * 256; }
+}  // namespace
+
+// In 2-D the slowest waves are only about twice the others, and the second
+// launch (4 us) costs as much as it saves: 100,000 box queries of 100,000
+// points on a circle, k = 8 522 -> 453 us, but 160,000 queries of 16 uniform
+// clouds 75 -> 79.
+size_t tail_workspace_bytes(int64_t total_q, int D) {
+    return D == 2 ? 0 : tail_masks_bytes(total_q) + static_cast<size_t>(total_q) * 4;
+}
+
+void set_tail(KnnArgs& a, void* ws) {
+    a.tail_masks = static_cast<uint64_t*>(ws);
+    a.tail_bounds = reinterpret_cast<float*>(static_cast<char*>(ws) + tail_masks_bytes(a.total_q));
+    a.tail_budget = tail_budget(a.total_q);
+}
+
+namespace {
 // Workspace: the cells' first-point tables (a routed search's second
 // structure's after the first's), the clouds' flags (B, or 2B routed), the
 // two failure lists' counts (kGridCounts each, kCountStride words apart),
@@ -1899,7 +1890,18 @@ hipError_t launch_grid_knn(const KnnArgs& args, const float* node_aabbs, int64_t
     f.fb_bound = bounds;
     f.fb_count = passes == 2 ? counts2 : counts;
     f.fb_seg = g.seg;
-    return launch_knn_accel(f, D, K, false, stream);
+    if (tail_workspace_bytes(args.total_q, D) == 0) return launch_knn_accel(f, D, K, false, stream);
+    // The queries it gives up: masks in the list that is not in use (a
+    // work-group's 64 entries of it hold its mask), bounds in place.
+    f.node_aabbs = node_aabbs;
+    f.num_real_nodes = static_cast<int32_t>(nr);
+    f.node_aabbs2 = node_aabbs2;
+    f.num_real_nodes2 = static_cast<int32_t>(nr2);
+    f.tail_masks = reinterpret_cast<uint64_t*>(passes == 2 ? list : list2);
+    f.tail_bounds = bounds;
+    f.tail_budget = tail_budget(args.total_q);
+    if ((e = launch_knn_accel(f, D, K, false, stream)) != hipSuccess) return e;
+    return launch_knn_tail(f, D, K, false, stream);
 }
 
 }  // namespace tbvh

@@ -17,7 +17,7 @@
 // List.  One key per lane, ascending over the lanes: the 64 smallest keys
 // seen (the first K are the result).  The first four blocks (64 points,
 // nearest first) fill it by one bitonic sort over the lanes; later points
-// below the k-th key wait in LDS and are merged 64 at a time.  Keys and
+// below the k-th key are inserted, or merged 64 at a time.  Keys and
 // distances are the traversal's, so the result is the same k smallest
 // (distance, index) pairs, bit for bit; a box is skipped only when its
 // distance exceeds the k-th distance.
@@ -27,6 +27,8 @@
 // time against the traversal: 1,000 queries of 50,000 3-D points at k = 8
 // 73 -> 23 us, 10,000 of 10,000 at k = 4 64 -> 31 us (kernel); which calls take
 // it: WAVE_MAX_QUERIES in _native.py.
+#include <algorithm>
+
 #include "knn_common.hpp"
 
 namespace tbvh {
@@ -34,7 +36,7 @@ namespace {
 
 constexpr int kBlockBits = 4;   // points per block: 16
 constexpr int kFanBits = 6;     // levels per step: 64 children
-constexpr int kMergeAt = 32;    // pending candidates that trigger a merge
+constexpr int kInsertMost = 24; // accepted keys of a step inserted one by one
 
 template <int kCtrl>
 __device__ __forceinline__ uint64_t dpp_key(uint64_t k) {
@@ -90,6 +92,18 @@ __device__ __forceinline__ uint64_t reversed64(uint64_t k) {
     uint64_t even, odd;
     pair_keys<false>(reversed32(k), even, odd);
     return (lane_id() & 32) ? even : odd;
+}
+
+// key_max with a wave-uniform second operand.
+__device__ __forceinline__ uint64_t key_max_uniform(uint64_t a, uint64_t b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(__longlong_as_double(a)), "s"(__longlong_as_double(b)));
+    return static_cast<uint64_t>(__double_as_longlong(r));
+}
+
+// The next lower lane's key; lane 0 reads 0.
+__device__ __forceinline__ uint64_t shifted(uint64_t k) {
+    return dpp_key<0x138>(k);  // wave_shr:1
 }
 
 // Bitonic sequence over the 64 lanes -> ascending.
@@ -154,12 +168,25 @@ struct WaveQuery {
     const float4* pts;    // this cloud's Morton-ordered points
     int n, L, vl, bl;     // points, leaf level, virtual leaves, block level
     float q[D];
-    uint64_t* pend;       // candidates waiting for a merge (128 keys of LDS)
-    int waiting;          // how many (wave-uniform)
     bool filled;          // the first blocks are in the list
     uint64_t list;        // this lane's key, ascending over the lanes
-    uint64_t kth;         // key of lane K - 1 (wave-uniform)
+    uint64_t kth;         // key of lane K - 1, or the starting bound's (wave-uniform)
     float worst;          // its distance
+
+    // `bound`: at least K points lie within it (kFar: unknown).
+    __device__ __forceinline__ void init(const float* nodes_, const float4* pts_, int n_, float bound) {
+        nodes = nodes_;
+        pts = pts_;
+        n = n_;
+        L = tree::leaf_level(n);
+        vl = tree::virtual_leaves(n);
+        bl = L > kBlockBits ? L - kBlockBits : 0;
+        filled = false;
+        // Entries (bound, -1) in every lane: K points displace those below K.
+        list = candidate_key(bound, 0xffffffffu);
+        kth = list;
+        worst = bound;
+    }
 
     __device__ __forceinline__ void set_kth() {
         const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(list), K - 1);
@@ -168,14 +195,24 @@ struct WaveQuery {
         worst = __uint_as_float(hi);
     }
 
-    __device__ __forceinline__ void merge() {
-        __builtin_amdgcn_wave_barrier();
-        for (int base = 0; base < waiting; base += kWave) {
-            const uint64_t k = base + lane_id() < waiting ? pend[base + lane_id()] : kEmptyKey;
-            list = clean64(key_min(list, reversed64(sort64(k))));
+    // Adds the lanes' keys below the k-th one (`in`, the lanes of mask `m`).
+    // Few are inserted one by one: the lanes from the key's rank on take
+    // their lower neighbour's, 6 instructions (a key past the k-th by then
+    // lands past lane K - 1).  Many are sorted over the lanes and merged:
+    // the smaller of list and reversed keys is a bitonic sequence of the 64
+    // smallest (28 exchanges, about 200 instructions).
+    __device__ __forceinline__ void add(uint64_t key, bool in, uint64_t m) {
+        if (__popcll(m) > kInsertMost) {
+            list = clean64(key_min(list, reversed64(sort64(in ? key : kEmptyKey))));
+        } else {
+            do {
+                const int from = __builtin_ctzll(m);
+                m &= m - 1;
+                const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(key), from);
+                const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(key >> 32), from);
+                list = key_min(list, key_max_uniform(shifted(list), (static_cast<uint64_t>(hi) << 32) | lo));
+            } while (m != 0);
         }
-        __builtin_amdgcn_wave_barrier();
-        waiting = 0;
         set_kth();
     }
 
@@ -200,15 +237,14 @@ struct WaveQuery {
         while (mask != 0) {
             // Four blocks, 16 lanes each: the nearest four while the list is
             // empty, then in storage order.
-            int mine = -1;
+            int b[4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                if (mask != 0) {
-                    const int b = filled ? __ffsll(static_cast<long long>(mask)) - 1 : nearest_lane(d, mask);
-                    mask &= ~(1ull << b);
-                    if ((lane_id() >> 4) == g) mine = first + b;
-                }
+                b[g] = mask == 0 ? -1 : filled ? static_cast<int>(__builtin_ctzll(mask)) : nearest_lane(d, mask);
+                mask = mask == 0 ? 0 : mask & ~(1ull << b[g]);
             }
+            const int pick = lane_id() < 32 ? (lane_id() < 16 ? b[0] : b[1]) : (lane_id() < 48 ? b[2] : b[3]);
+            const int mine = pick < 0 ? -1 : first + pick;
             const int at = (mine << bits) + slot;
             const bool valid = mine >= 0 && slot < (1 << bits) && at < n;
             const float4 p = pts[valid ? at : 0];
@@ -216,18 +252,13 @@ struct WaveQuery {
             const uint64_t key = valid && dist < kFar ? candidate_key(dist, __float_as_uint(p.w)) : kEmptyKey;
             if (!filled) {
                 filled = true;
-                list = sort64(key);
+                list = key_min(list, sort64(key));
                 set_kth();
             } else {
                 const bool in = key < kth;
                 const uint64_t m = __ballot(in);
                 if (m == 0) continue;
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
-                                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
-                if (in) pend[waiting + rank] = key;
-                waiting += __popcll(m);
-                if (waiting < kMergeAt) continue;
-                merge();
+                add(key, in, m);
             }
             mask &= __ballot(d <= worst);
         }
@@ -248,79 +279,142 @@ struct WaveQuery {
                 const int c = nearest_lane(d, mask);
                 expand<kBelow - 1>(first + c);
                 mask &= ~(1ull << c);
-                // The candidates still waiting tighten the bound before the
-                // next run's boxes are read.
-                if (mask != 0 && waiting > 0) merge();
                 mask &= __ballot(d <= worst);
             }
         }
     }
 };
 
-template <int D, int K, int kSteps>
-__global__ __launch_bounds__(kWave) void knn_wave_kernel(KnnArgs a) {
-    __shared__ uint64_t s_pend[kMergeAt + kWave];
-    const int64_t gid = blockIdx.x;
-    const int64_t seg = gid / a.M;
-    const int64_t local = gid - seg * a.M;
-    const int64_t qi = a.order != nullptr ? a.order[gid] : local;
-    if (qi < 0 || qi >= a.M) return;  // a corrupt order never indexes out of range
-    const int64_t row = seg * a.M + qi;
-    const int64_t pstart = seg * a.num_leaves;
-    WaveQuery<D, K> w;
-    w.nodes = a.node_aabbs + seg * a.num_real_nodes * (2 * D);
-    w.pts = static_cast<const float4*>(a.accel) + pstart;
-    w.n = a.num_leaves;
-    w.L = tree::leaf_level(w.n);
-    w.vl = tree::virtual_leaves(w.n);
-    w.bl = w.L > kBlockBits ? w.L - kBlockBits : 0;
-#pragma unroll
-    for (int d = 0; d < D; ++d) w.q[d] = a.queries[row * D + d];
-    w.pend = s_pend;
-    w.waiting = 0;
-    w.filled = false;
-    w.list = kEmptyKey;
-    w.kth = kEmptyKey;
-    w.worst = kFar;
-    w.template expand<kSteps - 1>(0);
-    if (w.waiting > 0) w.merge();
+// Wide steps from a top level of at most 64 nodes down to the blocks: four
+// cover the accel's largest cloud (2^28 points).
+__host__ __device__ inline int wave_steps(int n) {
+    const int L = tree::leaf_level(n);
+    const int bl = L > kBlockBits ? L - kBlockBits : 0;
+    return bl <= kFanBits ? 1 : (bl + kFanBits - 1) / kFanBits;
+}
 
-    if (lane_id() < K) {
-        const int64_t out_row = a.spatial_output ? gid : row;
-        const int64_t idx = static_cast<int32_t>(static_cast<uint32_t>(w.list));
-        a.out_indices[out_row * K + lane_id()] = idx;
-        a.out_distances[out_row * K + lane_id()] = __uint_as_float(static_cast<uint32_t>(w.list >> 32));
-        if (a.out_positions != nullptr) {
-            const int C = a.source_cols;
-            float* op = a.out_positions + (out_row * K + lane_id()) * C;
-            const float* src = a.source_points + (pstart + (idx >= 0 ? idx : 0)) * C;
-            for (int c = 0; c < C; ++c) op[c] = idx >= 0 ? src[c] : 0.0f;
+// The list's first K entries (and their rows) into result row `out_row`.
+template <int D, int K>
+__device__ __forceinline__ void write_list(const KnnArgs& a, uint64_t list, int64_t out_row, int64_t index_offset,
+                                           int64_t pstart) {
+    if (lane_id() >= K) return;
+    const int64_t idx = static_cast<int32_t>(static_cast<uint32_t>(list));
+    a.out_indices[out_row * K + lane_id()] = idx >= 0 ? idx + index_offset : idx;
+    a.out_distances[out_row * K + lane_id()] = __uint_as_float(static_cast<uint32_t>(list >> 32));
+    if (a.out_positions != nullptr) {
+        const int C = a.source_cols;
+        float* op = a.out_positions + (out_row * K + lane_id()) * C;
+        const float* src = a.source_points + (pstart + (idx >= 0 ? idx : 0)) * C;
+        for (int c = 0; c < C; ++c) op[c] = idx >= 0 ? src[c] : 0.0f;
+    }
+}
+
+// kSteps: wave_steps(l.n), or 0 to look it up.
+template <int D, int K, int kSteps>
+__device__ __forceinline__ void wave_search(const KnnArgs& a, const QueryLoc& l, float bound) {
+    WaveQuery<D, K> w;
+    w.init((l.second ? a.node_aabbs2 : a.node_aabbs) + l.nstart * (2 * D),
+           static_cast<const float4*>(l.second ? a.accel2 : a.accel) + l.pstart, l.n, bound);
+#pragma unroll
+    for (int d = 0; d < D; ++d) w.q[d] = a.queries[l.row * D + d];
+    switch (kSteps > 0 ? kSteps : wave_steps(l.n)) {
+        case 1: w.template expand<0>(0); break;
+        case 2: w.template expand<1>(0); break;
+        case 3: w.template expand<2>(0); break;
+        default: w.template expand<3>(0); break;
+    }
+    write_list<D, K>(a, w.list, l.out_row, l.index_offset, l.pstart);
+}
+
+// The plain call has a kernel for each number of steps: a lone wave's time is
+// partly its cold instruction fetches (1,000 queries of 50,000 points 28 us with
+// the number looked up, 24 us without).
+template <int D, int K, bool kOrdered, bool kRagged, int kSteps>
+__global__ __launch_bounds__(kWave) void knn_wave_kernel(KnnArgs a) {
+    const QueryLoc l = locate<kOrdered, kRagged, false, false>(a, blockIdx.x);
+    if (l.row < 0) return;  // a corrupt order never indexes out of range
+    wave_search<D, K, kSteps>(a, l, kFar);
+}
+
+// The queries that the traversal's waves gave up (KnnArgs::tail_masks), one
+// after the other per wave.  Work-group b takes lane b % 64 of every
+// stride-th traversal work-group, so queries given up together, by one wave
+// or by its neighbours, go to different work-groups (four lanes per work-group
+// read the marks in 5 us instead of 6 at 18,400 work-groups, but the routed
+// search of 357,000 queries of surface clouds went 1.7 -> 4.4 ms).
+template <int D, int K, bool kOrdered, bool kRagged, bool kRouted>
+__global__ __launch_bounds__(kWave) void knn_tail_kernel(KnnArgs a, int groups) {
+    const int stride = static_cast<int>(gridDim.x) / kWave;
+    const int slot = static_cast<int>(blockIdx.x) % kWave;
+    for (int first = static_cast<int>(blockIdx.x) / kWave; first < groups; first += stride * kWave) {
+        const int g = first + lane_id() * stride;
+        const uint64_t mask = g < groups ? a.tail_masks[g] : 0;
+        uint64_t todo = __ballot((mask >> slot) & 1ull);
+        while (todo != 0) {
+            const int block = first + __builtin_ctzll(todo) * stride;
+            todo &= todo - 1;
+            // The launch position of lane `slot` of that work-group, as in
+            // the traversal.
+            const int xcd = block % kXcds, rest = block / kXcds;
+            int64_t gid = (static_cast<int64_t>(xcd) * (groups / kXcds) + rest) * kKnnBlock + slot;
+            if (a.fb_list != nullptr) {
+                const int sub = xcd * kGridSubLists + rest % kGridSubLists;
+                gid = a.fb_list[sub * a.fb_seg + static_cast<int64_t>(rest / kGridSubLists) * kKnnBlock + slot];
+            }
+            const QueryLoc l = locate<kOrdered, kRagged, kRouted, false>(a, gid);
+            if (l.row >= 0) wave_search<D, K, 0>(a, l, a.tail_bounds[gid]);
         }
     }
 }
 
 template <int D, int K>
-void launch_steps(const KnnArgs& a, hipStream_t stream) {
+void launch_wave(const KnnArgs& a, bool ragged, hipStream_t stream) {
     const unsigned grid = static_cast<unsigned>(a.total_q);
-    // Wide steps from a top level of at most 64 nodes down to the blocks.
-    const int L = tree::leaf_level(a.num_leaves);
-    const int bl = L > kBlockBits ? L - kBlockBits : 0;
-    const int steps = bl <= kFanBits ? 1 : (bl + kFanBits - 1) / kFanBits;
-    switch (steps) {
-        case 1: knn_wave_kernel<D, K, 1><<<grid, kWave, 0, stream>>>(a); break;
-        case 2: knn_wave_kernel<D, K, 2><<<grid, kWave, 0, stream>>>(a); break;
-        case 3: knn_wave_kernel<D, K, 3><<<grid, kWave, 0, stream>>>(a); break;
-        default: knn_wave_kernel<D, K, 4><<<grid, kWave, 0, stream>>>(a); break;
+    const bool ordered = a.order != nullptr;
+    if (ragged && ordered) knn_wave_kernel<D, K, true, true, 0><<<grid, kWave, 0, stream>>>(a);
+    else if (ragged) knn_wave_kernel<D, K, false, true, 0><<<grid, kWave, 0, stream>>>(a);
+    else if (ordered) knn_wave_kernel<D, K, true, false, 0><<<grid, kWave, 0, stream>>>(a);
+    else switch (wave_steps(a.num_leaves)) {
+        case 1: knn_wave_kernel<D, K, false, false, 1><<<grid, kWave, 0, stream>>>(a); break;
+        case 2: knn_wave_kernel<D, K, false, false, 2><<<grid, kWave, 0, stream>>>(a); break;
+        case 3: knn_wave_kernel<D, K, false, false, 3><<<grid, kWave, 0, stream>>>(a); break;
+        default: knn_wave_kernel<D, K, false, false, 4><<<grid, kWave, 0, stream>>>(a); break;
     }
 }
 
 template <int D>
-hipError_t launch_k(const KnnArgs& a, int K, hipStream_t stream) {
+hipError_t launch_wave_k(const KnnArgs& a, int K, bool ragged, hipStream_t stream) {
     switch (K) {
-        case 4: launch_steps<D, 4>(a, stream); break;
-        case 8: launch_steps<D, 8>(a, stream); break;
-        case 16: launch_steps<D, 16>(a, stream); break;
-        case 32: launch_steps<D, 32>(a, stream); break;
+        case 4: launch_wave<D, 4>(a, ragged, stream); break;
+        case 8: launch_wave<D, 8>(a, ragged, stream); break;
+        case 16: launch_wave<D, 16>(a, ragged, stream); break;
+        case 32: launch_wave<D, 32>(a, ragged, stream); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+template <int D, int K>
+void launch_tail(const KnnArgs& a, bool ragged, hipStream_t stream) {
+    // The traversal's grid (knn.hip launch_dk); 64 work-groups per stride.
+    const int64_t tiles = (a.total_q + kKnnBlock - 1) / kKnnBlock;
+    const int groups = static_cast<int>((tiles + kXcds - 1) / kXcds * kXcds);
+    const unsigned grid = static_cast<unsigned>(std::min((groups + kWave - 1) / kWave, 128) * kWave);
+    const bool ordered = a.order != nullptr;
+    if (a.routes != nullptr) knn_tail_kernel<D, K, true, false, true><<<grid, kWave, 0, stream>>>(a, groups);
+    else if (ragged && ordered) knn_tail_kernel<D, K, true, true, false><<<grid, kWave, 0, stream>>>(a, groups);
+    else if (ragged) knn_tail_kernel<D, K, false, true, false><<<grid, kWave, 0, stream>>>(a, groups);
+    else if (ordered) knn_tail_kernel<D, K, true, false, false><<<grid, kWave, 0, stream>>>(a, groups);
+    else knn_tail_kernel<D, K, false, false, false><<<grid, kWave, 0, stream>>>(a, groups);
+}
+
+template <int D>
+hipError_t launch_tail_k(const KnnArgs& a, int K, bool ragged, hipStream_t stream) {
+    switch (K) {
+        case 4: launch_tail<D, 4>(a, ragged, stream); break;
+        case 8: launch_tail<D, 8>(a, ragged, stream); break;
+        case 16: launch_tail<D, 16>(a, ragged, stream); break;
+        case 32: launch_tail<D, 32>(a, ragged, stream); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -328,11 +422,14 @@ hipError_t launch_k(const KnnArgs& a, int K, hipStream_t stream) {
 
 }  // namespace
 
-hipError_t launch_knn_wave(const KnnArgs& a, int D, int K, hipStream_t stream) {
+hipError_t launch_knn_tail(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream) {
     if (a.total_q == 0) return hipSuccess;
-    // Four steps of six levels and the blocks' four cover 2^28 points.
-    if (a.num_leaves < 1 || a.num_leaves > kMaxAccelCloud) return hipErrorInvalidValue;
-    return D == 3 ? launch_k<3>(a, K, stream) : launch_k<2>(a, K, stream);
+    return D == 3 ? launch_tail_k<3>(a, K, ragged, stream) : launch_tail_k<2>(a, K, ragged, stream);
+}
+
+hipError_t launch_knn_wave(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream) {
+    if (a.total_q == 0) return hipSuccess;
+    return D == 3 ? launch_wave_k<3>(a, K, ragged, stream) : launch_wave_k<2>(a, K, ragged, stream);
 }
 
 }  // namespace tbvh

@@ -438,13 +438,29 @@ struct KnnArgs {
     const float* fb_bound;
     const uint32_t* fb_count;
     int64_t fb_seg;
+    // Tail (accel only; null: none): queries that a traversal wave gives up
+    // (see traverse) are marked in tail_masks[work-group], bit per lane, with
+    // their k-th distance so far in tail_bounds[launch position], and
+    // launch_knn_tail finishes them over node_aabbs (ragged: node_offsets;
+    // routed: node_aabbs2 for the false route).
+    uint64_t* tail_masks;
+    float* tail_bounds;
+    int32_t tail_budget;
 };
 hipError_t launch_knn(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream);
 hipError_t launch_knn_accel(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream);
 
-// Batched accel k-NN with one wave per query (knn_wave.hip; not routed):
-// reads the accel's points and node_aabbs.
-hipError_t launch_knn_wave(const KnnArgs& a, int D, int K, hipStream_t stream);
+// Accel k-NN with one wave per query (knn_wave.hip; not routed): reads the
+// accel's points and node_aabbs (ragged: node_offsets).
+hipError_t launch_knn_wave(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream);
+// The queries marked in a.tail_masks by launch_knn_accel with the same
+// arguments, one wave per query.
+hipError_t launch_knn_tail(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream);
+
+// Tail workspace of a traversal of total_q queries (0: no tail): the masks of
+// its work-groups, then the bounds (set_tail points `a` at them).
+size_t tail_workspace_bytes(int64_t total_q, int D);
+void set_tail(KnnArgs& a, void* ws);
 
 // Cell-block k-NN (batched accel, `a` as for launch_knn_accel; spatial
 // output and neighbour rows as there): every cloud's accel points are cut
