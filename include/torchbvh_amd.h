@@ -512,6 +512,16 @@ int tbvh_knn_accel_routed_grid_spatial(const void* true_accel, const float* true
 int tbvh_interpolate_neighbors(const float* values, const int64_t* indices, const float* weights,
                                const uint8_t* exact, int64_t B, int64_t N, int64_t H, int64_t C, int k,
                                float* out, void* stream);
+/* Gradient of tbvh_interpolate_neighbors' values: out (B, N, H, C) from the
+ * result's gradient `grad` (B, N, H, C); indices, weights and exact as there
+ * (indices outside [0, N) add nothing).  Sums in ascending (row, neighbour)
+ * order. */
+int tbvh_interpolate_backward_workspace_size(int64_t B, int64_t N, int64_t H, int k, size_t* bytes);
+int tbvh_interpolate_backward(const float* grad, const int64_t* indices, const float* weights,
+                              const uint8_t* exact, int64_t B, int64_t N, int64_t H, int64_t C,
+                              int k, float* out, void* workspace, size_t workspace_bytes,
+                              void* stream);
+
 
 #ifdef __cplusplus
 }

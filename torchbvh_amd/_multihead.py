@@ -21,6 +21,9 @@ from ._validation import check_cuda_f32, dense, dense_offsets
 __all__ = ["query_displaced_knn", "gather_neighbor_values", "interpolate_displaced"]
 
 
+_NOT_LOCAL = "gather_neighbor_values: indices must be local source indices"
+
+
 def _check_displaced(pos: torch.Tensor, q: torch.Tensor, op: str) -> None:
     """Shape, dtype and device checks of the displaced-query helpers
     (reference order and messages: _multihead.py:17-35)."""
@@ -89,11 +92,58 @@ def gather_neighbor_values(values: torch.Tensor, indices: torch.Tensor) -> torch
     if indices.numel() > 0:
         lo, hi = torch.aminmax(indices)
         if int(lo) < 0 or int(hi) >= values.size(1):
-            raise ValueError(f"{op}: indices must be local source indices")
+            raise ValueError(_NOT_LOCAL)
     B, _, H, _ = values.shape
     batch = torch.arange(B, device=values.device).view(B, 1, 1, 1)
     head = torch.arange(H, device=values.device).view(1, 1, H, 1)
     return values[batch, indices, head]
+
+
+class _Interpolate(torch.autograd.Function):
+    """`_C.interpolate_neighbors`, differentiable (any number of times) in its
+    values: the result is linear in them."""
+
+    @staticmethod
+    def forward(values, indices, weights, exact):
+        return _C.interpolate_neighbors(values.contiguous(), indices, weights, exact)
+
+    @staticmethod
+    def setup_context(ctx, inputs, output):
+        ctx.save_for_backward(*inputs[1:])
+
+    @staticmethod
+    def backward(ctx, grad):
+        return _InterpolateTransposed.apply(grad, *ctx.saved_tensors), None, None, None
+
+
+class _InterpolateTransposed(torch.autograd.Function):
+    """The gradient of `_Interpolate` in its values, itself linear."""
+
+    @staticmethod
+    def forward(grad, indices, weights, exact):
+        return _C.interpolate_neighbors_backward(grad.contiguous(), indices, weights, exact)
+
+    @staticmethod
+    def setup_context(ctx, inputs, output):
+        ctx.save_for_backward(*inputs[1:])
+
+    @staticmethod
+    def backward(ctx, grad):
+        return _Interpolate.apply(grad, *ctx.saved_tensors), None, None, None
+
+
+def _kernels_differentiate(values: torch.Tensor, indices: torch.Tensor) -> bool:
+    """Whether the differentiable call may run as the library's kernels: plain
+    tensors outside of every transform that has to see the tensor operations
+    (functorch levels, forward-mode, dispatch and function modes, tracing),
+    and entry counts the backward's sort can number."""
+    C = torch._C
+    return (type(values) in (torch.Tensor, torch.nn.Parameter)
+            and not C._functorch.is_functorch_wrapped_tensor(values)
+            and torch.autograd.forward_ad._current_level < 0
+            and C._len_torch_dispatch_stack() == 0 and C._len_torch_function_stack() == 0
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and 0 < indices.numel() <= 2**31 - 1)
 
 
 def interpolate_displaced(pos: torch.Tensor, q: torch.Tensor, values: torch.Tensor, k: int = 8, *,
@@ -120,13 +170,27 @@ def interpolate_displaced(pos: torch.Tensor, q: torch.Tensor, values: torch.Tens
     values = dense(values)
     indices, d2 = query_displaced_knn(dense(pos), dense(q), k, return_positions=False)
     eps = EXACT_DISTANCE_EPSILON
+    training = values.requires_grad and torch.is_grad_enabled()
+    fused = training and _kernels_differentiate(values, indices)
+    if fused:
+        # Missing neighbours (index -1, always a row's last entries) are
+        # refused below; the value is on its way to the host meanwhile.
+        least = indices[..., -1].amin().to("cpu", non_blocking=True)
+        arrived = torch.cuda.Event()
+        arrived.record(torch.cuda.current_stream(indices.device))
     exact = d2 <= eps
     weights = torch.reciprocal(d2 + eps)
     weights = weights / weights.sum(dim=-1, keepdim=True).clamp(min=eps)
-    if not (values.requires_grad and torch.is_grad_enabled()):
+    if not training:
         # One kernel: the same rank-by-rank sums and exact-hit select, with
         # no gathered copy and no host synchronisation.
         return _C.interpolate_neighbors(values, indices, weights, exact)
+    if fused:
+        out = _Interpolate.apply(values, indices, weights, exact)
+        arrived.synchronize()
+        if int(least) < 0:
+            raise ValueError(_NOT_LOCAL)
+        return out
     neighbours = gather_neighbor_values(values, indices)  # (B, N, H, k, Ch)
     # Accumulated neighbour rank by neighbour rank, the reference's order of
     # fp32 additions (_multihead.py:123-144).

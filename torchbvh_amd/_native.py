@@ -142,6 +142,10 @@ def _declare(L) -> None:
         [_vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _int, _int, _vp, _int, _vp, _vp, _vp, _vp]
     )
     L.tbvh_interpolate_neighbors.argtypes = [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _vp]
+    L.tbvh_interpolate_backward_workspace_size.argtypes = [_i64, _i64, _i64, _int, _szp]
+    L.tbvh_interpolate_backward.argtypes = (
+        [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _vp, ctypes.c_size_t, _vp]
+    )
     for name in (
         "tbvh_build_workspace_size", "tbvh_build", "tbvh_build_ragged_workspace_size",
         "tbvh_build_ragged", "tbvh_build_with_accel", "tbvh_build_ragged_with_accel",
@@ -159,7 +163,7 @@ def _declare(L) -> None:
         "tbvh_knn_accel_routed_grid_workspace_size", "tbvh_knn_accel_routed_grid_spatial",
         "tbvh_build_primitives_workspace_size", "tbvh_build_primitives",
         "tbvh_morton_sort_points_workspace_size", "tbvh_morton_sort_points",
-        "tbvh_interpolate_neighbors", "tbvh_build_with_accel_noalloc", "tbvh_accel_build_from_tree",
+        "tbvh_interpolate_neighbors", "tbvh_interpolate_backward_workspace_size", "tbvh_interpolate_backward", "tbvh_build_with_accel_noalloc", "tbvh_accel_build_from_tree",
     ):
         getattr(L, name).restype = _int
 
@@ -1108,6 +1112,32 @@ class _NativeOps:
             _check(load().tbvh_interpolate_neighbors(
                 _ptr(values), _ptr(indices), _ptr(weights), _ptr(exact), B, N, H, C, k, _ptr(out),
                 _stream(dev)))
+        return out
+
+    @staticmethod
+    def interpolate_neighbors_backward(grad, indices, weights, exact):
+        """Gradient of `interpolate_neighbors` in its values: grad (B, N, H, C),
+        the others as there.  Returns (B, N, H, C)."""
+        op = "interpolate_neighbors_backward"
+        _require_device_f32(op, grad, "grad")
+        _require_device_i64(op, indices, "indices")
+        _require_device_f32(op, weights, "weights")
+        _require(exact.dtype == torch.bool and exact.is_contiguous(), op, "exact must be a contiguous bool tensor")
+        B, N, H, C = (int(x) for x in grad.shape)
+        k = int(indices.size(-1))
+        for name, t in (("indices", indices), ("weights", weights), ("exact", exact)):
+            _require(tuple(t.shape) == (B, N, H, k) and t.device == grad.device, op,
+                     f"{name} must have shape (B, N, H, k) on the gradient's device")
+        out = torch.empty_like(grad)
+        if out.numel() == 0:
+            return out
+        L = load()
+        dev = grad.device
+        with torch.cuda.device(dev):
+            ws = _workspace(_size(L.tbvh_interpolate_backward_workspace_size, B, N, H, k), dev)
+            _check(L.tbvh_interpolate_backward(
+                _ptr(grad), _ptr(indices), _ptr(weights), _ptr(exact), B, N, H, C, k, _ptr(out), _ptr(ws),
+                ws.numel(), _stream(dev)))
         return out
 
 

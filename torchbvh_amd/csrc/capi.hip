@@ -1445,4 +1445,60 @@ int tbvh_interpolate_neighbors(const float* values, const int64_t* indices, cons
     return ok();
 }
 
+namespace {
+// The backward's scratch: the sort's, the sorted entries and the
+// coefficients.
+struct InterpolateLayout {
+    Layout sort;
+    size_t order, coef, total;
+};
+InterpolateLayout make_interpolate_layout(int64_t B, int64_t entries) {
+    InterpolateLayout l;
+    l.sort = make_layout(B, entries, 3, false);
+    l.order = l.sort.total;
+    l.coef = align_up(l.order + static_cast<size_t>(entries) * 8);
+    l.total = align_up(l.coef + static_cast<size_t>(entries) * 4);
+    return l;
+}
+
+// Sizes of the backward: every entry (query row, neighbour) has a signed
+// 32-bit number, and a row's channels one too.
+int check_interpolate_backward(const char* op, int64_t B, int64_t N, int64_t H, int64_t C, int k, int64_t& entries) {
+    if (B < 1 || N < 1 || H < 1 || C < 1 || k < 1) {
+        return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: need B, N, H, C and k >= 1", op);
+    }
+    if (__builtin_mul_overflow(B, N, &entries) || __builtin_mul_overflow(entries, H, &entries) ||
+        __builtin_mul_overflow(entries, static_cast<int64_t>(k), &entries) || entries > kMaxRows || C > kMaxRows) {
+        return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: B * N * H * k and C must fit in signed int32", op);
+    }
+    return TBVH_OK;
+}
+}  // namespace
+
+int tbvh_interpolate_backward_workspace_size(int64_t B, int64_t N, int64_t H, int k, size_t* bytes) {
+    const char* op = "tbvh_interpolate_backward_workspace_size";
+    if (!bytes) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: bytes is null", op);
+    int64_t entries = 0;
+    if (int r = check_interpolate_backward(op, B, N, H, 1, k, entries)) return r;
+    *bytes = make_interpolate_layout(B, entries).total;
+    return ok();
+}
+
+int tbvh_interpolate_backward(const float* grad, const int64_t* indices, const float* weights, const uint8_t* exact,
+                              int64_t B, int64_t N, int64_t H, int64_t C, int k, float* out, void* ws,
+                              size_t ws_bytes, void* stream_ptr) {
+    const char* op = "tbvh_interpolate_backward";
+    int64_t entries = 0;
+    if (int r = check_interpolate_backward(op, B, N, H, C, k, entries)) return r;
+    if (!grad || !indices || !weights || !exact || !out) {
+        return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: null input or output pointer", op);
+    }
+    const InterpolateLayout l = make_interpolate_layout(B, entries);
+    if (int r = check_workspace(op, ws, ws_bytes, l.total)) return r;
+    TBVH_TRY(op, launch_interpolate_backward(grad, indices, weights, exact, B, N, H, C, k, carve<Segment>(ws, l.sort.segs),
+                                             l.sort.tiles, sort_buffers(ws, l.sort), carve<int64_t>(ws, l.order),
+                                             carve<float>(ws, l.coef), out, static_cast<hipStream_t>(stream_ptr)));
+    return ok();
+}
+
 }  // extern "C"

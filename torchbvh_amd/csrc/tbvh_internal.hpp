@@ -395,6 +395,14 @@ hipError_t launch_interpolate(const float* values, const int64_t* indices, const
                               const uint8_t* exact, int64_t rows, int64_t N, int64_t H, int64_t C, int K,
                               float* out, hipStream_t stream);
 
+// Gradient of its values: `out` (B * N * H, C) from the result's gradient.
+// Sort scratch as for launch_sort over B clouds of N * H * K entries, with
+// `order` and `coef` one word per entry.
+hipError_t launch_interpolate_backward(const float* grad, const int64_t* indices, const float* weights,
+                                       const uint8_t* exact, int64_t B, int64_t N, int64_t H, int64_t C, int K,
+                                       Segment* segs, int64_t tiles, const SortBuffers& sb, int64_t* order,
+                                       float* coef, float* out, hipStream_t stream);
+
 // k-NN traversal.
 struct KnnArgs {
     const float* node_aabbs;
