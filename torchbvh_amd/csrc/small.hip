@@ -12,6 +12,19 @@
 // ascending original index (the CUB contract the sort replaces,
 // bvh_build.cu:580-594), and the bounds are the same fminf/fmaxf reductions
 // from the same seeds (bvh_build.cu:453-494).
+//
+// The order is that of the unique pairs (key, row), so it need not be reached
+// by stable passes.  First the keys are dealt to bins by their top bits, each
+// bin's keys to as many sub-bins as it holds keys by the next bits (two rounds
+// of LDS counters and a scan each, about a key to a sub-bin wherever the
+// density is smooth at the scale of a bin), and a key's place in its sub-bin is
+// counted from the pairs there.  Only when a sub-bin holds more than
+// kMostInBin keys (many equal codes) do the four stable passes run, whose
+// ballot ranking (about 90 instructions per key and pass) bounds them on the one
+// CU.  Point ordering by passes and by bins, us: 4,000 3-D points 25 and 15,
+// 10,000 53 and 27, in eight clusters 52 and 34; the bins' attempt costs a cloud of a
+// few distinct points that then takes the passes 3 to 5 us (10,000 of 64: 50 and
+// 55; a limit of 96 keys: 4,000 of 64 24 and 52).
 #include "tbvh_internal.hpp"
 
 namespace tbvh {
@@ -19,6 +32,42 @@ namespace {
 
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallWaves = kSmallThreads / kWave;
+
+constexpr uint32_t kMostInBin = 32;
+
+// 16-bit counters, two to an LDS word (a cloud has fewer than 2^16 rows).
+__device__ __forceinline__ uint32_t count_half(uint32_t* words, uint32_t i) {
+    const uint32_t shift = (i & 1u) * 16u;
+    return (atomicAdd(&words[i >> 1], 1u << shift) >> shift) & 0xffffu;
+}
+__device__ __forceinline__ uint32_t read_half(const uint32_t* words, uint32_t i) {
+    return reinterpret_cast<const uint16_t*>(words)[i];
+}
+
+// Counters (kPer per thread, in order) -> their exclusive prefix sums, with
+// the total after the last one.  Starts and ends with a barrier.
+template <int kPer>
+__device__ __forceinline__ void scan_halves(uint32_t* words, uint32_t* scratch) {
+    static_assert(kPer % 2 == 0, "whole words per thread");
+    __syncthreads();
+    uint32_t w[kPer / 2];
+    uint32_t sum = 0;
+#pragma unroll
+    for (int i = 0; i < kPer / 2; ++i) {
+        w[i] = words[threadIdx.x * (kPer / 2) + i];
+        sum += (w[i] & 0xffffu) + (w[i] >> 16);
+    }
+    uint32_t total = 0;
+    uint32_t run = block_exclusive_sum<kSmallThreads>(sum, scratch, &total);
+#pragma unroll
+    for (int i = 0; i < kPer / 2; ++i) {
+        const uint32_t second = run + (w[i] & 0xffffu);
+        words[threadIdx.x * (kPer / 2) + i] = run | second << 16;
+        run = second + (w[i] >> 16);
+    }
+    if (threadIdx.x == 0) words[kSmallThreads * (kPer / 2)] = total;
+    __syncthreads();
+}
 
 // One cloud per work-group (segment blockIdx.x).  The cloud's rows are dealt
 // to all the waves in contiguous ranges of `per_wave` rows (a multiple of
@@ -36,9 +85,17 @@ __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
     float* __restrict__ scene_max, bool bounds, float seed_lo, float seed_hi, int first_bit, int passes,
     int64_t* __restrict__ order, uint32_t* __restrict__ sorted_keys) {
     constexpr int kCap = kItems * kSmallThreads;
+    // Bins: about one per key of a full cloud.
+    constexpr int kBinBits = kItems <= 4 ? 12 : 14;
+    constexpr int kBins = 1 << kBinBits;
+    constexpr int kPassWords = kSmallWaves * kRadix;
+    constexpr int kBinWords = kBins / 2 + 1;
     __shared__ uint32_t s_keys[kCap];
-    __shared__ uint32_t s_vals[kCap];
-    __shared__ uint32_t s_cnt[kSmallWaves][kRadix];
+    // The passes' values; by bins, the rows (16 bits each) and the sub-bins.
+    __shared__ uint32_t s_vals[kCap + 1];
+    // The passes' digit counters; by bins, the bins.
+    __shared__ uint32_t s_count[kPassWords > kBinWords ? kPassWords : kBinWords];
+    uint32_t (*s_cnt)[kRadix] = reinterpret_cast<uint32_t (*)[kRadix]>(s_count);
     __shared__ uint32_t s_start[kRadix];
     __shared__ uint32_t s_scan[kSmallWaves];
     __shared__ float s_red[kSmallWaves][2 * D];
@@ -107,9 +164,83 @@ __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
         for (int u = 0; u < kChunk; ++u) {
             const int i = c + u;
             const int j = base + i * kWave;
-            key[i] = valid(i) ? (kHilbert ? hilbert::schedule_key<D>(r[u].v, lo, hi) : morton::encode<D>(r[u].v, lo, hi))
+            // The bits below first_bit (the schedule's key holds two in 3-D) take
+            // no part in the order.
+            key[i] = valid(i) ? (kHilbert ? hilbert::schedule_key<D>(r[u].v, lo, hi) >> first_bit << first_bit
+                                          : morton::encode<D>(r[u].v, lo, hi))
                               : 0xffffffffu;
             val[i] = static_cast<uint32_t>(j);
+        }
+    }
+
+    {
+        constexpr int kLow = morton::key_bits<D>() - kBinBits;  // bits below a bin's
+        static_assert(kLow >= 14, "a bin's sub-bins take at most log2(kSmallCloud) bits");
+        uint32_t* bins = s_count;
+        uint32_t* sub = s_vals;
+        uint16_t* rows16 = reinterpret_cast<uint16_t*>(s_vals + kCap / 2 + 1);
+        for (int i = threadIdx.x; i < kBinWords; i += kSmallThreads) bins[i] = 0u;
+        for (int i = threadIdx.x; i < kCap / 2 + 1; i += kSmallThreads) sub[i] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            if (valid(i)) count_half(bins, key[i] >> kLow);
+        }
+        scan_halves<kBins / kSmallThreads>(bins, s_scan);
+        // A bin of c keys from place s has its floor-log2(c)-bit sub-bins at
+        // counters s .. s + c - 1.
+        uint32_t at[kItems];
+        uint32_t most = 0;
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            if (valid(i)) {
+                const uint32_t b = key[i] >> kLow;
+                const uint32_t first = read_half(bins, b);
+                const int m = 31 - __builtin_clz(read_half(bins, b + 1) - first);
+                const uint32_t slot = first + ((key[i] >> (kLow - m)) & ((1u << m) - 1u));
+                const uint32_t arrived = count_half(sub, slot);
+                at[i] = slot | arrived << 16;
+                most = max(most, arrived);
+            }
+        }
+        if (!__syncthreads_or(most >= kMostInBin)) {
+            scan_halves<kItems>(sub, s_scan);
+#pragma unroll
+            for (int i = 0; i < kItems; ++i) {
+                if (valid(i)) {
+                    const uint32_t place = read_half(sub, at[i] & 0xffffu) + (at[i] >> 16);
+                    s_keys[place] = key[i];
+                    rows16[place] = static_cast<uint16_t>(val[i]);
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kItems; ++i) {
+                if (valid(i)) {
+                    const uint32_t slot = at[i] & 0xffffu;
+                    const uint32_t first = read_half(sub, slot), end = read_half(sub, slot + 1);
+                    uint32_t place = first;
+                    for (uint32_t j = first; j < end; ++j) {
+                        const uint32_t k = s_keys[j];
+                        place += k < key[i] || (k == key[i] && rows16[j] < val[i]) ? 1u : 0u;
+                    }
+                    at[i] = place;
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kItems; ++i) {
+                if (valid(i)) {
+                    s_keys[at[i]] = key[i];
+                    rows16[at[i]] = static_cast<uint16_t>(val[i]);
+                }
+            }
+            __syncthreads();
+            for (int j = threadIdx.x; j < n; j += kSmallThreads) {
+                order[g.start + j] = static_cast<int64_t>(rows16[j]);
+                if (sorted_keys) sorted_keys[g.start + j] = s_keys[j];
+            }
+            return;
         }
     }
 
