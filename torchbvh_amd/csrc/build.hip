@@ -251,7 +251,7 @@ __global__ __launch_bounds__(kTileThreads) void morton_kernel(const float* __res
     const Segment g = first_launch_segment(segs, S, plan, t, &s_seg, &s);
     const int lt = static_cast<int>(t - g.tile_first);
     if (lt >= g.tiles) {
-        if (tile_hist && threadIdx.x < kRadix) tile_hist[threadIdx.x * tstride + t] = 0u;
+        if (tile_hist && threadIdx.x < kRadix) tile_hist[hist_at(threadIdx.x, t, tstride)] = 0u;
         return;
     }
     const int64_t row0 = g.start + static_cast<int64_t>(lt) * kSortTile;
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(kTileThreads) void morton_kernel(const float* __res
         }
     }
     __syncthreads();
-    if (tile_hist && threadIdx.x < kRadix) tile_hist[threadIdx.x * tstride + t] = s_hist[threadIdx.x];
+    if (tile_hist && threadIdx.x < kRadix) tile_hist[hist_at(threadIdx.x, t, tstride)] = s_hist[threadIdx.x];
 }
 
 // ---------------------------------------------------------------------------

@@ -156,7 +156,7 @@ hipError_t run_build(const float* points, const int64_t* offsets, int64_t S, int
                      int64_t rows, int D, const BuildOut& o, void* ws, hipStream_t stream, int V = 0) {
     const Layout l = make_layout(S, rows, D, true, V > 0);
     Segment* segs = carve<Segment>(ws, l.segs);
-    const SortBuffers sb = sort_buffers(ws, l);
+    SortBuffers sb = sort_buffers(ws, l);
     const bool ragged = offsets != nullptr;
     // Equal clouds of points need no planning launch: the bounds kernel
     // computes their segments and stores the table for the later launches.
@@ -175,6 +175,7 @@ hipError_t run_build(const float* points, const int64_t* offsets, int64_t S, int
     // Bounds reduced inside the Morton kernel unless a cloud may span more
     // than kFuseBoundsTiles tiles (ragged: bounded by all rows).
     const int64_t cloud_bound = ragged ? rows : n_uniform;
+    sb.tstride = sort_tstride(cloud_bound, sb.tstride);
     const bool fuse = (cloud_bound + kSortTile - 1) / kSortTile <= kFuseBoundsTiles;
     // The point build seeds its bounds at +-1e30 (bvh_build.cu:466-467);
     // the primitive build (the boxes' min/max, bvh_build.cu:60-93) and the
@@ -255,7 +256,8 @@ hipError_t run_query_sort(const float* queries, const int64_t* offsets, int64_t 
                           hipStream_t stream) {
     const Layout l = make_layout(S, rows, D, false);
     Segment* segs = carve<Segment>(ws, l.segs);
-    const SortBuffers sb = sort_buffers(ws, l);
+    SortBuffers sb = sort_buffers(ws, l);
+    sb.tstride = sort_tstride(offsets ? rows : m_uniform, sb.tstride);
     // Equal clouds need no planning launch: the Morton kernel computes their
     // segments and stores the table for the sort.
     UniformPlan plan;
@@ -1495,8 +1497,10 @@ int tbvh_interpolate_backward(const float* grad, const int64_t* indices, const f
     }
     const InterpolateLayout l = make_interpolate_layout(B, entries);
     if (int r = check_workspace(op, ws, ws_bytes, l.total)) return r;
+    SortBuffers sb = sort_buffers(ws, l.sort);
+    sb.tstride = sort_tstride(entries / B, sb.tstride);
     TBVH_TRY(op, launch_interpolate_backward(grad, indices, weights, exact, B, N, H, C, k, carve<Segment>(ws, l.sort.segs),
-                                             l.sort.tiles, sort_buffers(ws, l.sort), carve<int64_t>(ws, l.order),
+                                             l.sort.tiles, sb, carve<int64_t>(ws, l.order),
                                              carve<float>(ws, l.coef), out, static_cast<hipStream_t>(stream_ptr)));
     return ok();
 }

@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kBlock) void interpolate_keys_kernel(const int64_t*
         atomicAdd(&s_cnt[key & (kRadix - 1)], 1u);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < kRadix; i += kBlock) tile_hist[i * tstride + blockIdx.x] = s_cnt[i];
+    for (int i = threadIdx.x; i < kRadix; i += kBlock) tile_hist[hist_at(i, blockIdx.x, tstride)] = s_cnt[i];
 }
 
 // One thread per V channels of a target row: its run of sorted entries, found

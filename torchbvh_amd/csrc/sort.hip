@@ -13,7 +13,8 @@
 //   1. count: each tile's digit counts, digit-major [digit][tile] (for the
 //      first pass the key producer writes them: launch_morton /
 //      launch_route_keys);
-//   2. scan: one work-group per digit, exclusive scan along the tiles;
+//   2. scan: one work-group per digit, exclusive scan along the tiles (not
+//      for clouds of few tiles, whose scatter sums the counts itself);
 //   3. scatter: each tile ranks its keys stably (wave64 ballot matching),
 //      takes its segment-relative digit offsets from the scan
 //      (scan[d][t] - scan[d][first tile of the segment]) and the segment's
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(kThreads) void tile_count_kernel(const Segment* __r
         }
     }
     __syncthreads();
-    if (threadIdx.x < kRadix) tile_hist[threadIdx.x * tstride + t] = s_cnt[threadIdx.x];
+    if (threadIdx.x < kRadix) tile_hist[hist_at(threadIdx.x, t, tstride)] = s_cnt[threadIdx.x];
 }
 
 // Exclusive scan of one digit's tile counts along the tiles (work-group
@@ -101,7 +102,9 @@ __global__ __launch_bounds__(kScanThreads) void tile_scan_kernel(const uint32_t*
     }
 }
 
-template <bool kFirst, bool kLast>
+// kInline: the tile sums its cloud's digit counts itself (tile_hist, tile-
+// major), and no scan is launched (sort_sums_inline).
+template <bool kFirst, bool kLast, bool kInline>
 __global__ __launch_bounds__(kThreads) void scatter_kernel(const Segment* __restrict__ segs, int S,
                                                            SortPass pass) {
     __shared__ int s_seg;
@@ -143,7 +146,30 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(const Segment* __rest
     // segment before this one and the segment's total.
     const int d = threadIdx.x;
     uint32_t before_tiles = 0, seg_count = 0;
-    if (d < kRadix) {
+    if constexpr (kInline) {
+        // Each digit's column by two threads, one for every other eight
+        // tiles; eight counts at a time, loaded together (past the cloud's
+        // last tile its first is read and not added).
+        static_assert(kThreads == 2 * kRadix, "two threads per digit");
+        const int digit = d & (kRadix - 1);
+        const uint32_t* col = pass.tile_hist + static_cast<int64_t>(g.tile_first) * kRadix + digit;
+        for (int j0 = d < kRadix ? 0 : 8; j0 < g.tiles; j0 += 16) {
+            uint32_t c[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) c[j] = col[(j0 + j < g.tiles ? j0 + j : 0) * kRadix];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t in = j0 + j < g.tiles ? c[j] : 0u;
+                seg_count += in;
+                before_tiles += j0 + j < lt ? in : 0u;
+            }
+        }
+        if (d >= kRadix) {
+            s_base[digit] = seg_count;
+            s_start[digit] = before_tiles;
+            seg_count = 0;
+        }
+    } else if (d < kRadix) {
         const uint32_t* col = pass.tile_scan + d * pass.tstride;
         const uint32_t seg0 = col[g.tile_first];
         before_tiles = col[t] - seg0;
@@ -167,6 +193,10 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(const Segment* __rest
     // The tile's count of digit d and the waves' offsets within it.
     uint32_t tile_count = 0;
     if (d < kRadix) {
+        if constexpr (kInline) {
+            seg_count += s_base[d];
+            before_tiles += s_start[d];
+        }
         uint32_t run = 0;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
@@ -226,11 +256,18 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(const Segment* __rest
     }
 }
 
+template <bool kFirst, bool kLast>
+void launch_scatter(bool in_line, unsigned grid, const Segment* segs, int S, const SortPass& pass, hipStream_t stream) {
+    if (in_line) scatter_kernel<kFirst, kLast, true><<<grid, kThreads, 0, stream>>>(segs, S, pass);
+    else scatter_kernel<kFirst, kLast, false><<<grid, kThreads, 0, stream>>>(segs, S, pass);
+}
+
 }  // namespace
 
 hipError_t launch_sort(const Segment* segs, int64_t S, int64_t tiles, SortBits bits,
                        const SortBuffers& b, int64_t* order, uint32_t* sorted_keys,
                        hipStream_t stream) {
+    const bool in_line = b.tstride == 0;
     const unsigned grid = static_cast<unsigned>(tiles);
     const int passes = bits.passes();
     const int Si = static_cast<int>(S);
@@ -243,7 +280,9 @@ hipError_t launch_sort(const Segment* segs, int64_t S, int64_t tiles, SortBits b
         if (p > 0) {
             tile_count_kernel<<<grid, kThreads, 0, stream>>>(segs, Si, kin, shift, b.tile_hist, b.tstride);
         }
-        tile_scan_kernel<<<kRadix, kScanThreads, 0, stream>>>(b.tile_hist, b.tile_scan, tiles, b.tstride);
+        if (!in_line) {
+            tile_scan_kernel<<<kRadix, kScanThreads, 0, stream>>>(b.tile_hist, b.tile_scan, tiles, b.tstride);
+        }
         SortPass pass;
         pass.keys_in = kin;
         pass.vals_in = vin;
@@ -251,20 +290,16 @@ hipError_t launch_sort(const Segment* segs, int64_t S, int64_t tiles, SortBits b
         pass.vals_out = vout;
         pass.idx_out = order;
         pass.tile_scan = b.tile_scan;
+        pass.tile_hist = b.tile_hist;
         pass.tstride = b.tstride;
         pass.shift = shift;
         const bool first = p == 0;
         const bool last = p == passes - 1;
         if (last) pass.keys_out = sorted_keys;
-        if (first && last) {
-            scatter_kernel<true, true><<<grid, kThreads, 0, stream>>>(segs, Si, pass);
-        } else if (first) {
-            scatter_kernel<true, false><<<grid, kThreads, 0, stream>>>(segs, Si, pass);
-        } else if (last) {
-            scatter_kernel<false, true><<<grid, kThreads, 0, stream>>>(segs, Si, pass);
-        } else {
-            scatter_kernel<false, false><<<grid, kThreads, 0, stream>>>(segs, Si, pass);
-        }
+        if (first && last) launch_scatter<true, true>(in_line, grid, segs, Si, pass, stream);
+        else if (first) launch_scatter<true, false>(in_line, grid, segs, Si, pass, stream);
+        else if (last) launch_scatter<false, true>(in_line, grid, segs, Si, pass, stream);
+        else launch_scatter<false, false>(in_line, grid, segs, Si, pass, stream);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         uint32_t* tk = kin; kin = kout; kout = tk;

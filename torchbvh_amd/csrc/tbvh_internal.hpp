@@ -219,6 +219,23 @@ struct SortBuffers {
     int64_t tstride;      // >= tiles_bound, a multiple of 64
 };
 
+// With tstride 0 the counts are tile-major ([tile][digit]) and every scatter
+// work-group sums its cloud's itself; tile_scan is not used.
+__host__ __device__ inline int64_t hist_at(int digit, int64_t tile, int64_t tstride) {
+    return tstride > 0 ? digit * tstride + tile : tile * kRadix + digit;
+}
+
+// The row stride for a sort of clouds of at most max_n rows: 0 up to
+// kInlineTiles tiles, whose work-groups then each read 1 KB of counts per tile of
+// the cloud, in place of one scan launch per pass.  Measured, point ordering with
+// scans / without, us: 50,000 points (13 tiles) 65 / 53, 131,072 (32) 67 / 56,
+// 262,144 (64) 68 / 61, 400,000 (98) 71 / 66, 524,288 (128) 72.6 / 71.4; 32 x 65,536
+// 113 / 99.
+constexpr int64_t kInlineTiles = 112;
+inline int64_t sort_tstride(int64_t max_n, int64_t tstride) {
+    return (max_n + kSortTile - 1) / kSortTile <= kInlineTiles ? 0 : tstride;
+}
+
 // Row stride of the digit-major tile arrays.
 inline int64_t tile_stride(int64_t tiles_bound) { return (tiles_bound + 63) / 64 * 64; }
 
@@ -230,6 +247,7 @@ struct SortPass {
     uint32_t* vals_out;
     int64_t* idx_out;
     const uint32_t* tile_scan;  // [digit][tile], exclusive along tiles
+    const uint32_t* tile_hist;  // [tile][digit] counts (inline sums)
     int64_t tstride;
     int shift;
 };
