@@ -182,6 +182,11 @@ int tbvh_sort_queries(const float* queries, int64_t B, int64_t M, int D,
                       int64_t* order,
                       void* workspace, size_t workspace_bytes, void* stream);
 
+/* out (B + 1) = the offsets if they rise strictly from 0 to `total`, else an
+ * even division of the rows (B <= total): ragged calls launched with `out`
+ * before the host has read the offsets stay inside their tensors. */
+int tbvh_safe_offsets(const int64_t* offsets, int64_t B, int64_t total, int64_t* out, void* stream);
+
 /* Ragged form: queries [total_q, D] packed by `query_offsets` (device int64
  * [B+1]); `order` [total_q] receives local query indices per cloud.  Replaces
  * the per-segment calls made by `_query_knn_ragged` (torchbvh/_query.py:347-360). */

@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import math
 import threading
 import weakref
 from pathlib import Path
@@ -142,6 +143,7 @@ def _declare(L) -> None:
         [_vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _int, _int, _vp, _int, _vp, _vp, _vp, _vp]
     )
     L.tbvh_interpolate_neighbors.argtypes = [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _vp]
+    L.tbvh_safe_offsets.argtypes = [_vp, _i64, _i64, _vp, _vp]
     L.tbvh_interpolate_backward_workspace_size.argtypes = [_i64, _i64, _i64, _int, _szp]
     L.tbvh_interpolate_backward.argtypes = (
         [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _vp, ctypes.c_size_t, _vp]
@@ -163,7 +165,7 @@ def _declare(L) -> None:
         "tbvh_knn_accel_routed_grid_workspace_size", "tbvh_knn_accel_routed_grid_spatial",
         "tbvh_build_primitives_workspace_size", "tbvh_build_primitives",
         "tbvh_morton_sort_points_workspace_size", "tbvh_morton_sort_points",
-        "tbvh_interpolate_neighbors", "tbvh_interpolate_backward_workspace_size", "tbvh_interpolate_backward", "tbvh_build_with_accel_noalloc", "tbvh_accel_build_from_tree",
+        "tbvh_safe_offsets", "tbvh_interpolate_neighbors", "tbvh_interpolate_backward_workspace_size", "tbvh_interpolate_backward", "tbvh_build_with_accel_noalloc", "tbvh_accel_build_from_tree",
     ):
         getattr(L, name).restype = _int
 
@@ -626,21 +628,26 @@ class _NativeOps:
         return order
 
     @staticmethod
-    def build_bvh_ragged(points: torch.Tensor, batch_offsets: torch.Tensor,
-                         counts: list[int], *, with_accel: bool = False) -> dict:
-        """Segmented build of packed clouds; `counts` are the host-side cloud
-        sizes (already validated).  Returns packed tensors and per-cloud node
-        offsets; with `with_accel` (and every cloud <= MAX_ACCEL_CLOUD) also
-        the acceleration structure under "accel" (None otherwise)."""
-        op = "build_bvh_ragged"
-        _require_device_f32(op, points, "points")
-        _require_device_i64(op, batch_offsets, "batch_offsets")
+    def safe_offsets(offsets: torch.Tensor, total: int) -> torch.Tensor:
+        """A copy of (B + 1,) int64 offsets on the device, replaced by an even
+        division of the `total` rows if they are not strictly increasing from
+        0 to `total` (at least B rows): what a launch before the host has seen
+        the offsets may index with."""
+        op = "safe_offsets"
+        _require_device_i64(op, offsets, "offsets")
+        out = torch.empty_like(offsets)
+        dev = offsets.device
+        with torch.cuda.device(dev):
+            _check(load().tbvh_safe_offsets(_ptr(offsets), int(offsets.numel()) - 1, int(total), _ptr(out),
+                                            _stream(dev)))
+        return out
+
+    @staticmethod
+    def _launch_ragged_build(points, batch_offsets, total_nodes: int, with_accel: bool) -> dict:
         L = load()
         T, D = (int(s) for s in points.shape)
-        B = len(counts)
+        B = int(batch_offsets.numel()) - 1
         dev = points.device
-        node_counts = [real_node_count(c) for c in counts]
-        total_nodes = sum(node_counts)
         with torch.cuda.device(dev):
             ws_bytes = _size(L.tbvh_build_ragged_workspace_size, B, T, D)
             node_aabbs = torch.empty((total_nodes, 2 * D), dtype=torch.float32, device=dev)
@@ -653,7 +660,7 @@ class _NativeOps:
             node_offsets = torch.empty(B + 1, dtype=torch.int64, device=dev)
             ws = _workspace(ws_bytes, dev)
             accel = None
-            if with_accel and max(counts) <= MAX_ACCEL_CLOUD:
+            if with_accel:
                 accel = torch.empty(_size(L.tbvh_accel_size, B, T, D), dtype=torch.uint8,
                                     device=dev)
                 _check(L.tbvh_build_ragged_with_accel(
@@ -667,11 +674,6 @@ class _NativeOps:
                     _ptr(sorted_indices), _ptr(scene_min), _ptr(scene_max), _ptr(left),
                     _ptr(right), _ptr(leaf), _ptr(node_offsets), total_nodes,
                     _ptr(ws), ws.numel(), _stream(dev)))
-        if accel is not None:
-            _record_accel(accel, node_aabbs, T)
-        host_node_offsets = [0]
-        for c in node_counts:
-            host_node_offsets.append(host_node_offsets[-1] + c)
         return {
             "node_aabbs": node_aabbs,
             "sorted_indices": sorted_indices,
@@ -681,9 +683,53 @@ class _NativeOps:
             "right_child_mem": right,
             "mem_to_leaf": leaf,
             "node_offsets": node_offsets,
-            "host_node_offsets": host_node_offsets,
             "accel": accel,
         }
+
+    @classmethod
+    def build_bvh_ragged(cls, points: torch.Tensor, batch_offsets: torch.Tensor,
+                         counts: list[int], *, with_accel: bool = False) -> dict:
+        """Segmented build of packed clouds; `counts` are the host-side cloud
+        sizes (already validated).  Returns packed tensors and per-cloud node
+        offsets; with `with_accel` (and every cloud <= MAX_ACCEL_CLOUD) also
+        the acceleration structure under "accel" (None otherwise)."""
+        op = "build_bvh_ragged"
+        _require_device_f32(op, points, "points")
+        _require_device_i64(op, batch_offsets, "batch_offsets")
+        total_nodes = sum(real_node_count(c) for c in counts)
+        packed = cls._launch_ragged_build(points, batch_offsets, total_nodes,
+                                          with_accel and max(counts) <= MAX_ACCEL_CLOUD)
+        return cls.trim_ragged_build(packed, counts)
+
+    @classmethod
+    def build_bvh_ragged_bounded(cls, points: torch.Tensor, batch_offsets: torch.Tensor) -> dict:
+        """The launch of `build_bvh_ragged` (with the accel) before the host
+        has seen the offsets: over `safe_offsets`, with node arrays for the
+        most nodes that B clouds of T points in total can have - 2n - 1 each
+        and at most log2(n) more, whose sum is largest for equal clouds.  For
+        `trim_ragged_build` once the offsets have passed; B <= T <=
+        MAX_ACCEL_CLOUD."""
+        op = "build_bvh_ragged"
+        _require_device_f32(op, points, "points")
+        T, B = int(points.size(0)), int(batch_offsets.numel()) - 1
+        most = 2 * T - B + int(B * math.log2(T / B)) + 1
+        return cls._launch_ragged_build(points, cls.safe_offsets(batch_offsets, T), most, True)
+
+    @staticmethod
+    def trim_ragged_build(packed: dict, counts: list[int]) -> dict:
+        """`packed` with its node arrays cut to the nodes that clouds of these
+        sizes have and the clouds' node offsets added; records the accel."""
+        host_node_offsets = [0]
+        for c in counts:
+            level = (c - 1).bit_length()
+            host_node_offsets.append(host_node_offsets[-1] + 2 * c - 1 + bin((1 << level) - c).count("1"))
+        total = host_node_offsets[-1]
+        for key in ("node_aabbs", "left_child_mem", "right_child_mem", "mem_to_leaf"):
+            packed[key] = packed[key][:total]
+        packed["host_node_offsets"] = host_node_offsets
+        if packed["accel"] is not None:
+            _record_accel(packed["accel"], packed["node_aabbs"], sum(counts))
+        return packed
 
     @staticmethod
     def build_accel(points: torch.Tensor, data: dict) -> torch.Tensor | None:

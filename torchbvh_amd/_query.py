@@ -14,16 +14,16 @@ import torch
 
 from ._constants import SUPPORTED_DIMS
 from ._handles import BVHHandle, BatchedBVHHandle, RaggedBVHHandle, live_payload
-from ._native import _C
+from ._native import MAX_ACCEL_CLOUD, _C
 from ._validation import (
+    OffsetsRead,
     check_build_extent,
     check_cuda_f32,
     check_k,
-    check_offsets,
-    check_ragged_points,
     check_source_points,
     dense,
     dense_offsets,
+    read_ragged_points,
 )
 
 
@@ -68,32 +68,53 @@ def _build_bvh_batched(points: torch.Tensor) -> BatchedBVHHandle:
 def _build_bvh_ragged(points: torch.Tensor, batch_offsets: torch.Tensor) -> RaggedBVHHandle:
     points = dense(points)
     batch_offsets = dense_offsets(batch_offsets)
-    offsets = check_ragged_points("build_bvh", points, batch_offsets)
-    check_build_extent("build_bvh", points)
-    counts = [b - a for a, b in zip(offsets, offsets[1:])]
-    packed = _C.build_bvh_ragged(points, batch_offsets, counts, with_accel=True)
+    read = read_ragged_points("build_bvh", points, batch_offsets)
+    total, clouds = int(points.size(0)), int(batch_offsets.numel()) - 1
+    if clouds <= total <= MAX_ACCEL_CLOUD:
+        # The build is launched while the offsets travel to the host, over a
+        # copy of them made safe on the device, and its result kept once they
+        # have passed (waiting first left the GPU idle about 50 us per call).
+        packed = _C.build_bvh_ragged_bounded(points, batch_offsets)
+        offsets = read.values()
+        counts = [b - a for a, b in zip(offsets, offsets[1:])]
+        packed = _C.trim_ragged_build(packed, counts)
+    else:
+        offsets = read.values()
+        check_build_extent("build_bvh", points)
+        counts = [b - a for a, b in zip(offsets, offsets[1:])]
+        packed = _C.build_bvh_ragged(points, batch_offsets, counts, with_accel=True)
     accel = packed["accel"]
     dim = int(points.size(1))
     node_offsets = packed["host_node_offsets"]
+    node_counts = [b - a for a, b in zip(node_offsets, node_offsets[1:])]
+    # Every cloud's views of the packed tensors, in one call per tensor.
+    views = zip(
+        packed["node_aabbs"].split(node_counts),
+        packed["sorted_indices"].split(counts),
+        packed["scene_min"].unbind(),
+        packed["scene_max"].unbind(),
+        packed["left_child_mem"].split(node_counts),
+        packed["right_child_mem"].split(node_counts),
+        packed["mem_to_leaf"].split(node_counts),
+    )
     handles = []
-    for b, n in enumerate(counts):
-        n0, n1 = node_offsets[b], node_offsets[b + 1]
-        p0, p1 = offsets[b], offsets[b + 1]
+    for n, nr, (nodes, order, lo, hi, left, right, leaf) in zip(counts, node_counts, views):
+        level = (n - 1).bit_length()
         handles.append(
             BVHHandle(
                 {
-                    "node_aabbs": packed["node_aabbs"][n0:n1],
-                    "sorted_indices": packed["sorted_indices"][p0:p1],
-                    "scene_min": packed["scene_min"][b],
-                    "scene_max": packed["scene_max"][b],
+                    "node_aabbs": nodes,
+                    "sorted_indices": order,
+                    "scene_min": lo,
+                    "scene_max": hi,
                     "num_leaves": n,
-                    "num_real_nodes": n1 - n0,
-                    "leaf_level": (n - 1).bit_length(),
-                    "virtual_leaves": (1 << (n - 1).bit_length()) - n,
+                    "num_real_nodes": nr,
+                    "leaf_level": level,
+                    "virtual_leaves": (1 << level) - n,
                     "dim": dim,
-                    "left_child_mem": packed["left_child_mem"][n0:n1],
-                    "right_child_mem": packed["right_child_mem"][n0:n1],
-                    "mem_to_leaf": packed["mem_to_leaf"][n0:n1],
+                    "left_child_mem": left,
+                    "right_child_mem": right,
+                    "mem_to_leaf": leaf,
                 }
             )
         )
@@ -250,31 +271,46 @@ def _query_knn_ragged(
         raise ValueError("query_knn: query_points must be on the same device as the BVH")
     queries = dense(query_points)
     query_offsets = dense_offsets(query_offsets)
-    q_offsets = check_offsets(
-        "query_knn", query_offsets, total_rows=int(queries.size(0)), device=queries.device
-    )
-    if len(q_offsets) - 1 != data["batch_size"]:
-        raise ValueError("query_knn: query_offsets batch size must match BVH batch_size")
+    total, clouds = int(queries.size(0)), int(data["batch_size"])
+    read = OffsetsRead("query_knn", query_offsets, total_rows=total, device=queries.device)
     p_offsets = bvh._aux["host_offsets"]
-    if any(b - a < k for a, b in zip(p_offsets, p_offsets[1:])):
-        raise ValueError("query_knn: each source sample must contain at least k points")
+
+    def check_rest() -> None:
+        if int(query_offsets.numel()) - 1 != clouds:
+            raise ValueError("query_knn: query_offsets batch size must match BVH batch_size")
+        if any(b - a < k for a, b in zip(p_offsets, p_offsets[1:])):
+            raise ValueError("query_knn: each source sample must contain at least k points")
+        if source_points is not None:
+            check_source_points("query_knn", "ragged", source_points, data, queries.device, p_offsets[-1])
+
+    # As in the build: with everything else in order the search is launched
+    # while the offsets travel, over a copy made safe on the device; what they
+    # are found to break is raised before anything else is.
+    try:
+        check_rest()
+    except ValueError:
+        read.values()
+        raise
+    if not clouds <= total <= 2**31 - 1:
+        read.values()
+    safe_offsets = _C.safe_offsets(query_offsets, total)
     if source_points is not None:
-        check_source_points("query_knn", "ragged", source_points, data, queries.device, p_offsets[-1])
         source_points = dense(source_points)
 
     packed = bvh._aux["packed"]
     order = None
-    if _schedule(True, int(queries.size(0))):
+    if _schedule(True, total):
         order = _C.morton_sort_queries_ragged(
-            queries, query_offsets, packed["scene_min"], packed["scene_max"], data["batch_size"],
-            schedule=True,
+            queries, safe_offsets, packed["scene_min"], packed["scene_max"], clouds, schedule=True,
         )
-    return _C.query_knn_ragged(
+    out = _C.query_knn_ragged(
         packed["node_aabbs"], packed["sorted_indices"], data["batch_offsets"],
-        packed["node_offsets"], queries, query_offsets, order, data["batch_size"],
+        packed["node_offsets"], queries, safe_offsets, order, clouds,
         data["dim"], k, accel=bvh._aux.get("accel"), total_points=p_offsets[-1],
         source_points=source_points,
     )
+    read.values()
+    return out
 
 
 def query_knn(

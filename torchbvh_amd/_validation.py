@@ -132,18 +132,38 @@ def check_cuda_f32(prefix: str, tensor: torch.Tensor, name: str) -> None:
     _walk(prefix, _CUDA_F32, tensor, name=name)
 
 
+class OffsetsRead:
+    """The values of a (B + 1,) int64 offsets tensor on their way to the host:
+    the tensor's own rules are checked here, the values' by `values()`, which
+    waits for the copy alone and not for what was launched after it."""
+
+    def __init__(self, prefix: str, offsets: torch.Tensor, *, total_rows: int, device: torch.device):
+        _walk(prefix, _OFFSETS_TENSOR, offsets, device)
+        self._prefix, self._total = prefix, total_rows
+        self._host = offsets.detach().to("cpu", non_blocking=True)
+        self._arrived = torch.cuda.Event()
+        self._arrived.record(torch.cuda.current_stream(offsets.device))
+
+    def values(self) -> list[int]:
+        self._arrived.synchronize()
+        values = self._host.tolist()
+        _walk(self._prefix, _OFFSETS_VALUES, values, self._total)
+        return values
+
+
 def check_offsets(prefix: str, offsets: torch.Tensor, *, total_rows: int, device: torch.device) -> list[int]:
     """Validate a (B + 1,) int64 offsets tensor and return its values as host
     ints (one device-to-host read)."""
-    _walk(prefix, _OFFSETS_TENSOR, offsets, device)
-    values = [int(v) for v in offsets.detach().cpu().tolist()]
-    _walk(prefix, _OFFSETS_VALUES, values, total_rows)
-    return values
+    return OffsetsRead(prefix, offsets, total_rows=total_rows, device=device).values()
+
+
+def read_ragged_points(prefix: str, points: torch.Tensor, offsets: torch.Tensor) -> OffsetsRead:
+    _walk(prefix, _RAGGED_POINTS, points, name="points")
+    return OffsetsRead(prefix, offsets, total_rows=int(points.size(0)), device=points.device)
 
 
 def check_ragged_points(prefix: str, points: torch.Tensor, offsets: torch.Tensor) -> list[int]:
-    _walk(prefix, _RAGGED_POINTS, points, name="points")
-    return check_offsets(prefix, offsets, total_rows=int(points.size(0)), device=points.device)
+    return read_ragged_points(prefix, points, offsets).values()
 
 
 def dense(tensor: torch.Tensor) -> torch.Tensor:

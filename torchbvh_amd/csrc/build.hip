@@ -53,6 +53,17 @@ __global__ __launch_bounds__(kBlock) void plan_uniform_kernel(Segment* segs, int
     store_uniform_table(segs, S, n, with_tree);
 }
 
+// One work-group: `out` = the offsets if they rise strictly from 0 to `total`,
+// else an even division of the `total` (>= S) rows, so that launches that run
+// before the host has read the offsets index inside their tensors.
+__global__ __launch_bounds__(kBlock) void safe_offsets_kernel(const int64_t* __restrict__ offsets, int64_t S,
+                                                              int64_t total, int64_t* __restrict__ out) {
+    bool bad = threadIdx.x == 0 && (offsets[0] != 0 || offsets[S] != total);
+    for (int64_t i = threadIdx.x; i < S; i += kBlock) bad = bad || offsets[i + 1] <= offsets[i];
+    const bool even = __syncthreads_or(bad);
+    for (int64_t i = threadIdx.x; i <= S; i += kBlock) out[i] = even ? i * total / S : offsets[i];
+}
+
 // One work-group scans all segments in chunks of kBlock.
 __global__ __launch_bounds__(kBlock) void plan_offsets_kernel(Segment* segs, const int64_t* offsets,
                                                               int64_t S, bool with_tree,
@@ -507,6 +518,11 @@ inline unsigned plan_grid(int64_t items) {
 
 hipError_t launch_plan_uniform(Segment* segs, int64_t S, int64_t n, bool tree, hipStream_t stream) {
     plan_uniform_kernel<<<plan_grid(S), kBlock, 0, stream>>>(segs, S, static_cast<int>(n), tree);
+    return hipGetLastError();
+}
+
+hipError_t launch_safe_offsets(const int64_t* offsets, int64_t S, int64_t total, int64_t* out, hipStream_t stream) {
+    safe_offsets_kernel<<<1, kBlock, 0, stream>>>(offsets, S, total, out);
     return hipGetLastError();
 }
 

@@ -1425,6 +1425,16 @@ int tbvh_knn_accel_routed_tail(const void* true_accel, const float* true_node_aa
     return ok();
 }
 
+int tbvh_safe_offsets(const int64_t* offsets, int64_t B, int64_t total, int64_t* out, void* stream_ptr) {
+    const char* op = "tbvh_safe_offsets";
+    if (B < 1 || total < B || total > kMaxRows) {
+        return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: need 1 <= B <= total rows <= INT32_MAX", op);
+    }
+    if (!offsets || !out) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: null input or output pointer", op);
+    TBVH_TRY(op, launch_safe_offsets(offsets, B, total, out, static_cast<hipStream_t>(stream_ptr)));
+    return ok();
+}
+
 int tbvh_interpolate_neighbors(const float* values, const int64_t* indices, const float* weights,
                                const uint8_t* exact, int64_t B, int64_t N, int64_t H, int64_t C, int k,
                                float* out, void* stream_ptr) {

@@ -253,6 +253,8 @@ struct SortPass {
 };
 
 
+hipError_t launch_safe_offsets(const int64_t* offsets, int64_t S, int64_t total, int64_t* out, hipStream_t stream);
+
 // Planning: fill the segment table.
 hipError_t launch_plan_uniform(Segment* segs, int64_t S, int64_t n, bool tree, hipStream_t stream);
 hipError_t launch_plan_offsets(Segment* segs, const int64_t* offsets, int64_t S, bool tree,
