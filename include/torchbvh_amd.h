@@ -199,6 +199,15 @@ int tbvh_sort_queries_ragged(const float* queries, const int64_t* query_offsets,
                              void* workspace, size_t workspace_bytes,
                              void* stream);
 
+/* The schedule of a search for k neighbours (the other arguments and the workspace as for
+ * the sorts above): `order` [B, M] or [total_q], local query indices per cloud, in
+ * nearly the order of the top 24 bits of the queries' Hilbert (k = 32) or Morton
+ * index; calls need not repeat it. */
+int tbvh_schedule_queries_fine(const float* queries, int64_t B, int64_t M, int D, int k,
+                               const float* scene_min, const float* scene_max,
+                               int64_t* order,
+                               void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- k-NN with neighbour rows (fused gather) ------------------------------------------
  * No entry-point counterpart: the reference gathers source_points[indices]
  * in Python after the k-NN call (torchbvh/_query.py:169-174, 203-215,

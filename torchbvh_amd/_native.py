@@ -76,6 +76,7 @@ def _declare(L) -> None:
     )
     L.tbvh_schedule_queries.argtypes = L.tbvh_sort_queries.argtypes
     L.tbvh_schedule_queries_ragged.argtypes = L.tbvh_sort_queries_ragged.argtypes
+    L.tbvh_schedule_queries_fine.argtypes = [_vp, _i64, _i64, _int, _int] + [_vp] * 4 + [ctypes.c_size_t, _vp]
     L.tbvh_sort_routed_queries_workspace_size.argtypes = [_i64, _i64, _int, _szp]
     L.tbvh_sort_routed_queries.argtypes = (
         [_vp, _vp, _i64, _i64, _int, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp]
@@ -154,6 +155,7 @@ def _declare(L) -> None:
         "tbvh_sort_queries_workspace_size", "tbvh_sort_queries",
         "tbvh_sort_queries_ragged_workspace_size", "tbvh_sort_queries_ragged",
         "tbvh_schedule_queries", "tbvh_schedule_queries_ragged",
+        "tbvh_schedule_queries_fine",
         "tbvh_morton_codes", "tbvh_knn", "tbvh_knn_ragged", "tbvh_accel_size",
         "tbvh_accel_workspace_size", "tbvh_accel_build", "tbvh_accel_build_ragged",
         "tbvh_knn_accel", "tbvh_knn_accel_ragged", "tbvh_knn_spatial", "tbvh_knn_accel_spatial",
@@ -780,10 +782,12 @@ class _NativeOps:
 
     @staticmethod
     def morton_sort_queries_narrow(queries: torch.Tensor, scene_min: torch.Tensor,
-                                   scene_max: torch.Tensor, *, schedule: bool = False) -> torch.Tensor:
+                                   scene_max: torch.Tensor, *, schedule: bool = False,
+                                   fine: int | None = None) -> torch.Tensor:
         """Stable Morton order of [B, M, D] queries against per-cloud bounds.
-        With ``schedule`` only the top 16 code bits are sorted (the
-        traversal schedule ``query_knn`` uses; results do not depend on it)."""
+        With ``schedule`` the order of the top 16 bits of Hilbert keys instead;
+        with ``fine`` = k too, the schedule ``query_knn`` uses, nearly the order of
+        24 bits and not the same on every call (results do not depend on it)."""
         op = "morton_sort_queries_narrow"
         _require_device_f32(op, queries, "queries")
         _require(scene_min.is_cuda and scene_max.is_cuda and scene_min.is_contiguous()
@@ -802,10 +806,13 @@ class _NativeOps:
         if M == 0:
             return order
         fn = L.tbvh_schedule_queries if schedule else L.tbvh_sort_queries
+        extra = ()
+        if schedule and fine is not None:
+            fn, extra = L.tbvh_schedule_queries_fine, (int(fine),)
         with torch.cuda.device(dev):
             ws_bytes = _size(L.tbvh_sort_queries_workspace_size, B, M, D)
             ws = _workspace(ws_bytes, dev)
-            _check(fn(_ptr(queries), B, M, D, _ptr(scene_min), _ptr(scene_max), _ptr(order),
+            _check(fn(_ptr(queries), B, M, D, *extra, _ptr(scene_min), _ptr(scene_max), _ptr(order),
                       _ptr(ws), ws.numel(), _stream(dev)))
         return order
 

@@ -169,6 +169,17 @@ def build_bvh(
 SCHEDULE_MIN_QUERIES = 1 << 17
 
 
+# From this many queries per cloud the schedule also orders the queries inside
+# a cell of its 16-bit keys (16 of them at a million).  Ordering and search of
+# uniform clouds, us, without / with: 2-D 4M k = 8 730 / 694, 3-D 1M k = 16 336 / 322;
+# 300,000 k = 8 213 / 222.
+FINE_MIN_QUERIES = 1 << 20
+
+
+def _fine(cloud_queries: int, k: int) -> dict:
+    return {"fine": k} if cloud_queries >= FINE_MIN_QUERIES else {}
+
+
 def _schedule(sort_queries: bool, total_queries: int) -> bool:
     return sort_queries and total_queries > SCHEDULE_MIN_QUERIES
 
@@ -200,7 +211,8 @@ def _query_knn_single(
         src = dense(source_points).unsqueeze(0)
     if _schedule(sort_queries, int(queries.size(1))):
         order = _C.morton_sort_queries_narrow(
-            queries, data["scene_min"].unsqueeze(0), data["scene_max"].unsqueeze(0), schedule=True
+            queries, data["scene_min"].unsqueeze(0), data["scene_max"].unsqueeze(0), schedule=True,
+            **_fine(int(queries.size(1)), k),
         )
         out = _C.query_knn_batched_cached_bounds_ordered(
             node_aabbs, sorted_indices, queries, order.contiguous(),
@@ -241,7 +253,7 @@ def _query_knn_batched(
         src = dense(source_points)
     if _schedule(sort_queries, int(queries.size(0) * queries.size(1))):
         order = _C.morton_sort_queries_narrow(queries, data["scene_min"], data["scene_max"],
-                                              schedule=True)
+                                              schedule=True, **_fine(int(queries.size(1)), k))
         return _C.query_knn_batched_cached_bounds_ordered(
             data["node_aabbs"], data["sorted_indices"], queries, order.contiguous(),
             data["num_leaves"], data["num_real_nodes"], data["dim"], k, accel=accel, source_points=src,

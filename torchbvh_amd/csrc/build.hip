@@ -241,7 +241,7 @@ __global__ __launch_bounds__(kBlock) void primitive_prep_kernel(const float* __r
 // ---------------------------------------------------------------------------
 // One work-group per tile (the sort's tiles).  Digit counts are gathered
 // with LDS atomics and stored digit-major; surplus tiles store zeros.
-template <int D, bool kHilbert>
+template <int D, int kCurve>
 __global__ __launch_bounds__(kTileThreads) void morton_kernel(const float* __restrict__ points,
                                                               const Segment* segs, int S,
                                                               float* __restrict__ scene_min,
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(kTileThreads) void morton_kernel(const float* __res
     for (int i = 0; i < kTileRows; ++i) {
         const int j = i * kTileThreads + threadIdx.x;
         if (j < count) {
-            const uint32_t code = kHilbert ? hilbert::schedule_key<D>(r[i].v, lo, hi) : morton::encode<D>(r[i].v, lo, hi);
+            const uint32_t code = hilbert::sort_key<D, kCurve>(r[i].v, lo, hi);
             keys[row0 + j] = code;
             if (tile_hist) atomicAdd(&s_hist[(code >> first_bit) & (kRadix - 1)], 1u);
         }
@@ -589,9 +589,13 @@ hipError_t launch_morton(const float* points, int D, const Segment* segs, int64_
                                                   tstride, bits.first_bit, fin, plan);
     };
     if (D == 3) {
-        bits.hilbert ? run(morton_kernel<3, true>) : run(morton_kernel<3, false>);
+        if (bits.curve == hilbert::kFine) run(morton_kernel<3, hilbert::kFine>);
+        else if (bits.curve == hilbert::kSchedule) run(morton_kernel<3, hilbert::kSchedule>);
+        else run(morton_kernel<3, hilbert::kMorton>);
     } else {
-        bits.hilbert ? run(morton_kernel<2, true>) : run(morton_kernel<2, false>);
+        if (bits.curve == hilbert::kFine) run(morton_kernel<2, hilbert::kFine>);
+        else if (bits.curve == hilbert::kSchedule) run(morton_kernel<2, hilbert::kSchedule>);
+        else run(morton_kernel<2, hilbert::kMorton>);
     }
     return hipGetLastError();
 }

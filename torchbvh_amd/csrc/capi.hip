@@ -129,7 +129,16 @@ int full_key_bits(int D) { return D == 3 ? 30 : 32; }
 // Digits of a full Morton sort, and of the traversal schedule (the top 16
 // bits of Hilbert keys on the same grid: two passes instead of four).
 SortBits full_sort(int D) { return SortBits{0, full_key_bits(D)}; }
-SortBits schedule_sort(int D) { return SortBits{full_key_bits(D) - 16, full_key_bits(D), true}; }
+SortBits schedule_sort(int D) { return SortBits{full_key_bits(D) - 16, full_key_bits(D), hilbert::kSchedule}; }
+// The finer schedule of the searches: 24 bits, of which the last eight are
+// ordered within each sort tile only (launch_refine), or all in a small sort.
+// Morton order, whose runs of 64 queries are the accel's own cells, except for
+// long searches: call of 1M points and queries, top 16 bits only / Hilbert / Morton,
+// us, sort included: surface near it k = 8 945 / 926 / 817, clusters themselves k = 16
+// 791 / 761 / 732, uniform 336 / 330 / 322, surface from its box k = 32 6019 / 6013 / 6390.
+SortBits fine_sort(int D, int k) {
+    return SortBits{full_key_bits(D) - 24, full_key_bits(D), k >= 32 ? hilbert::kFine : hilbert::kMorton, true};
+}
 
 // Everything one build call launches, in order: plan (+ clear), bounds
 // (primitive builds: boxes, centres and bounds), Morton (+ the first
@@ -271,6 +280,8 @@ hipError_t run_query_sort(const float* queries, const int64_t* offsets, int64_t 
         return launch_small_sort(queries, D, segs, S, plan, m_bound, const_cast<float*>(scene_min),
                                  const_cast<float*>(scene_max), false, 0.0f, 0.0f, bits, order, nullptr, stream);
     }
+    const bool refine = bits.refine;
+    if (refine) bits.first_bit = bits.end_bit - 16;  // two passes, then the tiles
     uint32_t* keys = codes_only ? codes_only : sb.keys_a;
     // Bounds given (BoundsFinish empty): the kernel only reads them.
     if ((e = launch_morton(queries, D, segs, S, l.tiles, const_cast<float*>(scene_min),
@@ -279,6 +290,10 @@ hipError_t run_query_sort(const float* queries, const int64_t* offsets, int64_t 
         return e;
     }
     if (codes_only) return hipSuccess;
+    if (refine) {
+        if ((e = launch_sort(segs, S, l.tiles, bits, sb, nullptr, nullptr, stream)) != hipSuccess) return e;
+        return launch_refine(segs, S, l.tiles, bits.end_bit, sb.keys_a, sb.vals_a, order, stream);
+    }
     return launch_sort(segs, S, l.tiles, bits, sb, order, nullptr, stream);
 }
 
@@ -571,7 +586,7 @@ int tbvh_sort_queries_workspace_size(int64_t B, int64_t M, int D, size_t* bytes)
 }
 
 static int sort_batched(const char* op, const float* queries, int64_t B, int64_t M, int D,
-                        const float* scene_min, const float* scene_max, bool schedule, int64_t* order,
+                        const float* scene_min, const float* scene_max, SortBits bits, int64_t* order,
                         uint32_t* codes, void* workspace, size_t workspace_bytes, void* stream_ptr) {
     if (int r = check_dim(op, D)) return r;
     if (B < 1 || M < 0) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: need B >= 1 and M >= 0", op);
@@ -584,7 +599,7 @@ static int sort_batched(const char* op, const float* queries, int64_t B, int64_t
     const Layout l = make_layout(B, B * M, D, false);
     if (int r = check_workspace(op, workspace, workspace_bytes, l.total)) return r;
     TBVH_TRY(op, run_query_sort(queries, nullptr, B, M, B * M, D, scene_min, scene_max,
-                                schedule ? schedule_sort(D) : full_sort(D), order, codes, workspace,
+                                bits, order, codes, workspace,
                                 static_cast<hipStream_t>(stream_ptr)));
     return ok();
 }
@@ -593,7 +608,7 @@ int tbvh_sort_queries(const float* queries, int64_t B, int64_t M, int D, const f
                       const float* scene_max, int64_t* order, void* workspace,
                       size_t workspace_bytes, void* stream_ptr) {
     if (!order && M > 0) return fail(TBVH_ERR_INVALID_ARGUMENT, "tbvh_sort_queries: null input or output pointer");
-    return sort_batched("tbvh_sort_queries", queries, B, M, D, scene_min, scene_max, false, order,
+    return sort_batched("tbvh_sort_queries", queries, B, M, D, scene_min, scene_max, full_sort(D), order,
                         nullptr, workspace, workspace_bytes, stream_ptr);
 }
 
@@ -601,7 +616,7 @@ int tbvh_schedule_queries(const float* queries, int64_t B, int64_t M, int D, con
                           const float* scene_max, int64_t* order, void* workspace,
                           size_t workspace_bytes, void* stream_ptr) {
     if (!order && M > 0) return fail(TBVH_ERR_INVALID_ARGUMENT, "tbvh_schedule_queries: null input or output pointer");
-    return sort_batched("tbvh_schedule_queries", queries, B, M, D, scene_min, scene_max, true, order,
+    return sort_batched("tbvh_schedule_queries", queries, B, M, D, scene_min, scene_max, schedule_sort(D), order,
                         nullptr, workspace, workspace_bytes, stream_ptr);
 }
 
@@ -609,7 +624,7 @@ int tbvh_morton_codes(const float* rows, int64_t B, int64_t M, int D, const floa
                       const float* scene_max, uint32_t* codes, void* workspace,
                       size_t workspace_bytes, void* stream_ptr) {
     if (!codes && M > 0) return fail(TBVH_ERR_INVALID_ARGUMENT, "tbvh_morton_codes: null input or output pointer");
-    return sort_batched("tbvh_morton_codes", rows, B, M, D, scene_min, scene_max, false, nullptr, codes,
+    return sort_batched("tbvh_morton_codes", rows, B, M, D, scene_min, scene_max, full_sort(D), nullptr, codes,
                         workspace, workspace_bytes, stream_ptr);
 }
 
@@ -625,7 +640,7 @@ int tbvh_sort_queries_ragged_workspace_size(int64_t B, int64_t total_q, int D, s
 
 static int sort_ragged(const char* op, const float* queries, const int64_t* query_offsets, int64_t B,
                        int64_t total_q, int D, const float* scene_min, const float* scene_max,
-                       bool schedule, int64_t* order, void* workspace, size_t workspace_bytes,
+                       SortBits bits, int64_t* order, void* workspace, size_t workspace_bytes,
                        void* stream_ptr) {
     if (int r = check_dim(op, D)) return r;
     if (B < 1 || total_q < 0) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: need B >= 1 and total_q >= 0", op);
@@ -637,7 +652,7 @@ static int sort_ragged(const char* op, const float* queries, const int64_t* quer
     const Layout l = make_layout(B, total_q, D, false);
     if (int r = check_workspace(op, workspace, workspace_bytes, l.total)) return r;
     TBVH_TRY(op, run_query_sort(queries, query_offsets, B, 0, total_q, D, scene_min, scene_max,
-                                schedule ? schedule_sort(D) : full_sort(D), order, nullptr, workspace,
+                                bits, order, nullptr, workspace,
                                 static_cast<hipStream_t>(stream_ptr)));
     return ok();
 }
@@ -647,7 +662,7 @@ int tbvh_sort_queries_ragged(const float* queries, const int64_t* query_offsets,
                              const float* scene_max, int64_t* order, void* workspace,
                              size_t workspace_bytes, void* stream_ptr) {
     return sort_ragged("tbvh_sort_queries_ragged", queries, query_offsets, B, total_q, D, scene_min,
-                       scene_max, false, order, workspace, workspace_bytes, stream_ptr);
+                       scene_max, full_sort(D), order, workspace, workspace_bytes, stream_ptr);
 }
 
 int tbvh_schedule_queries_ragged(const float* queries, const int64_t* query_offsets, int64_t B,
@@ -655,7 +670,16 @@ int tbvh_schedule_queries_ragged(const float* queries, const int64_t* query_offs
                                  const float* scene_max, int64_t* order, void* workspace,
                                  size_t workspace_bytes, void* stream_ptr) {
     return sort_ragged("tbvh_schedule_queries_ragged", queries, query_offsets, B, total_q, D,
-                       scene_min, scene_max, true, order, workspace, workspace_bytes, stream_ptr);
+                       scene_min, scene_max, schedule_sort(D), order, workspace, workspace_bytes, stream_ptr);
+}
+
+int tbvh_schedule_queries_fine(const float* queries, int64_t B, int64_t M, int D, int k, const float* scene_min,
+                               const float* scene_max, int64_t* order, void* workspace, size_t workspace_bytes,
+                               void* stream_ptr) {
+    const char* op = "tbvh_schedule_queries_fine";
+    if (!order && M > 0) return fail(TBVH_ERR_INVALID_ARGUMENT, "%s: null input or output pointer", op);
+    return sort_batched(op, queries, B, M, D, scene_min, scene_max, fine_sort(D, k), order, nullptr, workspace,
+                        workspace_bytes, stream_ptr);
 }
 
 // ---------------------------------------------------------------------------

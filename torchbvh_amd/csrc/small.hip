@@ -79,7 +79,7 @@ __device__ __forceinline__ void scan_halves(uint32_t* words, uint32_t* scratch) 
 // scene_min/max and keys the rows against it; otherwise scene_min/max are
 // read.  Passes sort 8-bit digits from first_bit up; the cloud-local order
 // goes to `order` (int64) and, if given, the sorted keys to `sorted_keys`.
-template <int D, int kItems, bool kHilbert>
+template <int D, int kItems, int kCurve>
 __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
     const float* __restrict__ rows, const Segment* segs, int S, UniformPlan plan, float* __restrict__ scene_min,
     float* __restrict__ scene_max, bool bounds, float seed_lo, float seed_hi, int first_bit, int passes,
@@ -166,9 +166,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
             const int j = base + i * kWave;
             // The bits below first_bit (the schedule's key holds two in 3-D) take
             // no part in the order.
-            key[i] = valid(i) ? (kHilbert ? hilbert::schedule_key<D>(r[u].v, lo, hi) >> first_bit << first_bit
-                                          : morton::encode<D>(r[u].v, lo, hi))
-                              : 0xffffffffu;
+            key[i] = valid(i) ? hilbert::sort_key<D, kCurve>(r[u].v, lo, hi) >> first_bit << first_bit : 0xffffffffu;
             val[i] = static_cast<uint32_t>(j);
         }
     }
@@ -314,15 +312,14 @@ void launch_items(const float* rows, const Segment* segs, int64_t S, UniformPlan
                   float* scene_max, bool bounds, float seed_lo, float seed_hi, SortBits bits, int64_t* order,
                   uint32_t* sorted_keys, hipStream_t stream) {
     const unsigned grid = static_cast<unsigned>(S);
-    if (bits.hilbert) {
-        small_sort_kernel<D, kItems, true><<<grid, kSmallThreads, 0, stream>>>(
-            rows, segs, static_cast<int>(S), plan, scene_min, scene_max, bounds, seed_lo, seed_hi, bits.first_bit,
-            bits.passes(), order, sorted_keys);
-    } else {
-        small_sort_kernel<D, kItems, false><<<grid, kSmallThreads, 0, stream>>>(
-            rows, segs, static_cast<int>(S), plan, scene_min, scene_max, bounds, seed_lo, seed_hi, bits.first_bit,
-            bits.passes(), order, sorted_keys);
-    }
+    const auto run = [&](auto kernel) {
+        kernel<<<grid, kSmallThreads, 0, stream>>>(rows, segs, static_cast<int>(S), plan, scene_min, scene_max, bounds,
+                                                   seed_lo, seed_hi, bits.first_bit, bits.passes(), order,
+                                                   sorted_keys);
+    };
+    if (bits.curve == hilbert::kFine) run(small_sort_kernel<D, kItems, hilbert::kFine>);
+    else if (bits.curve == hilbert::kSchedule) run(small_sort_kernel<D, kItems, hilbert::kSchedule>);
+    else run(small_sort_kernel<D, kItems, hilbert::kMorton>);
 }
 
 template <int D>
@@ -342,7 +339,80 @@ void launch_d(const float* rows, const Segment* segs, int64_t S, UniformPlan pla
     }
 }
 
+// The rows of one sort tile, already in order of their keys' top 16 bits, into
+// order of all their bits (nearly: rows of one slot stay in any order), for a
+// schedule, whose order changes no result.  Bins over the tile's key range and sub-bins as in
+// the small sort, by the key's place in the range.  One read and one write of 8
+// bytes a row: 9 us at 1M rows, 20 at 4M, where two more passes of the global sort
+// took 32 and 66.
+__global__ __launch_bounds__(kSmallThreads) void refine_kernel(const Segment* __restrict__ segs, int S, int key_bits,
+                                                               const uint32_t* __restrict__ keys,
+                                                               const uint32_t* __restrict__ vals,
+                                                               int64_t* __restrict__ order) {
+    constexpr int kItems = kSortTile / kSmallThreads;
+    static_assert(kItems % 2 == 0, "whole counter words per thread");
+    __shared__ uint32_t bins[kSortTile / 2 + 1];
+    __shared__ uint32_t sub[kSortTile / 2 + 1];
+    __shared__ uint32_t s_vals[kSortTile];
+    __shared__ uint32_t s_scan[kSmallWaves];
+    __shared__ int s_seg;
+    const int64_t t = blockIdx.x;
+    const int s = block_find_segment([&](int i) { return static_cast<int64_t>(segs[i].tile_first); }, S, t, &s_seg);
+    const Segment g = segs[s];
+    const int lt = static_cast<int>(t - g.tile_first);
+    if (lt >= g.tiles) return;  // surplus tile
+    const int64_t row0 = g.start + static_cast<int64_t>(lt) * kSortTile;
+    const int count = min(kSortTile, g.n - lt * kSortTile);
+    uint32_t key[kItems], val[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        const int j = i * kSmallThreads + threadIdx.x;
+        key[i] = keys[row0 + (j < count ? j : 0)];
+        val[i] = vals[row0 + (j < count ? j : 0)];
+    }
+    const uint32_t low = (1u << (key_bits - 16)) - 1u;
+    const uint32_t base = keys[row0] & ~low;
+    const float scale = static_cast<float>(kSortTile) / (static_cast<float>((keys[row0 + count - 1] | low) - base) + 1.0f);
+    for (int i = threadIdx.x; i < kSortTile / 2 + 1; i += kSmallThreads) {
+        bins[i] = 0u;
+        sub[i] = 0u;
+    }
+    __syncthreads();
+    float x[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        x[i] = fminf(static_cast<float>(key[i] - base) * scale, static_cast<float>(kSortTile - 1));
+        if (i * kSmallThreads + threadIdx.x < count) count_half(bins, static_cast<uint32_t>(x[i]));
+    }
+    scan_halves<kItems>(bins, s_scan);
+    uint32_t at[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        if (i * kSmallThreads + threadIdx.x < count) {
+            const uint32_t b = static_cast<uint32_t>(x[i]);
+            const uint32_t first = read_half(bins, b), held = read_half(bins, b + 1) - first;
+            const uint32_t slot = first + min(static_cast<uint32_t>((x[i] - static_cast<float>(b)) *
+                                                                    static_cast<float>(held)), held - 1u);
+            at[i] = slot | count_half(sub, slot) << 16;
+        }
+    }
+    scan_halves<kItems>(sub, s_scan);
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        if (i * kSmallThreads + threadIdx.x < count) s_vals[read_half(sub, at[i] & 0xffffu) + (at[i] >> 16)] = val[i];
+    }
+    __syncthreads();
+    for (int j = threadIdx.x; j < count; j += kSmallThreads) order[row0 + j] = static_cast<int64_t>(s_vals[j]);
+}
+
 }  // namespace
+
+hipError_t launch_refine(const Segment* segs, int64_t S, int64_t tiles, int key_bits, const uint32_t* keys,
+                         const uint32_t* vals, int64_t* order, hipStream_t stream) {
+    refine_kernel<<<static_cast<unsigned>(tiles), kSmallThreads, 0, stream>>>(segs, static_cast<int>(S), key_bits, keys,
+                                                                             vals, order);
+    return hipGetLastError();
+}
 
 hipError_t launch_small_sort(const float* rows, int D, const Segment* segs, int64_t S, UniformPlan plan,
                              int64_t max_n, float* scene_min, float* scene_max, bool bounds, float seed_lo,

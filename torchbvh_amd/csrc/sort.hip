@@ -294,7 +294,7 @@ hipError_t launch_sort(const Segment* segs, int64_t S, int64_t tiles, SortBits b
         pass.tstride = b.tstride;
         pass.shift = shift;
         const bool first = p == 0;
-        const bool last = p == passes - 1;
+        const bool last = p == passes - 1 && order != nullptr;
         if (last) pass.keys_out = sorted_keys;
         if (first && last) launch_scatter<true, true>(in_line, grid, segs, Si, pass, stream);
         else if (first) launch_scatter<true, false>(in_line, grid, segs, Si, pass, stream);

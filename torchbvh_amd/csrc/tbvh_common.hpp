@@ -204,6 +204,27 @@ TBVH_HD uint32_t schedule_key(const float* p, const float* lo, const float* hi) 
     return index<D, top>(x) << (D * (b - top));
 }
 
+// The top 24 bits of the Hilbert index (8 levels in 3-D, 12 in 2-D), in bits
+// [key_bits - 24, key_bits): schedule_key's with eight more bits.
+template <int D>
+TBVH_HD uint32_t fine_key(const float* p, const float* lo, const float* hi) {
+    constexpr int b = D == 3 ? 10 : 16;
+    constexpr int top = D == 3 ? 8 : 12;
+    uint32_t x[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) x[d] = morton::cell(morton::unit_coord(p[d], lo[d], hi[d]), 1u << b) >> (b - top);
+    return index<D, top>(x) << (D * (b - top));
+}
+
+// A sort's keys: Morton codes, the schedule's keys or its fine ones.
+enum Curve { kMorton = 0, kSchedule = 1, kFine = 2 };  // kFine: Hilbert
+template <int D, int kCurve>
+TBVH_HD uint32_t sort_key(const float* p, const float* lo, const float* hi) {
+    if constexpr (kCurve == kFine) return fine_key<D>(p, lo, hi);
+    else if constexpr (kCurve == kSchedule) return schedule_key<D>(p, lo, hi);
+    else return morton::encode<D>(p, lo, hi);
+}
+
 }  // namespace hilbert
 
 // ---------------------------------------------------------------------------

@@ -284,11 +284,12 @@ struct BoundsFinish {
 
 // Digit range of a sort: 8-bit digits at bits first_bit, first_bit + 8, ...
 // below end_bit (so passes = ceil((end_bit - first_bit) / 8) <= 4), and the
-// curve launch_morton keys rows on (Hilbert only for the query schedule).
+// curve launch_morton keys rows on (Hilbert only for the query schedules).
 struct SortBits {
     int first_bit;
     int end_bit;
-    bool hilbert = false;
+    hilbert::Curve curve = hilbert::kMorton;
+    bool refine = false;  // a schedule's: the bits below the top 16 within tiles
     int passes() const { return (end_bit - first_bit + kRadixBits - 1) / kRadixBits; }
 };
 
@@ -303,6 +304,12 @@ hipError_t launch_small_sort(const float* rows, int D, const Segment* segs, int6
                              int64_t max_n, float* scene_min, float* scene_max, bool bounds, float seed_lo,
                              float seed_hi, SortBits bits, int64_t* order, uint32_t* sorted_keys,
                              hipStream_t stream);
+
+// Sort tiles in order of their keys' top 16 of `key_bits` bits (an even number of
+// launch_sort passes without `order`: in buf.keys_a, buf.vals_a) into order of the
+// rest, tile by tile.
+hipError_t launch_refine(const Segment* segs, int64_t S, int64_t tiles, int key_bits, const uint32_t* keys,
+                         const uint32_t* vals, int64_t* order, hipStream_t stream);
 
 // Primitive BVH input: every primitive's box and centre, and each cloud's
 // bounds over the boxes (partials as in launch_bounds).
@@ -323,7 +330,8 @@ hipError_t launch_morton(const float* points, int D, const Segment* segs, int64_
 // Stable LSD sort of (key, local index) per segment on the digits of
 // `bits`; writes int64 local indices in key order into `order` and, if
 // `sorted_keys` is non-null, the keys in that order (an even number of
-// passes leaves them in buf.keys_a).  Input keys are in buf.keys_a
+// passes leaves them in buf.keys_a); without `order`, keys and u32 indices stay
+// in the buffers of the last pass.  Input keys are in buf.keys_a
 // (clobbered); buf.tile_hist holds the first digit's tile counts (written
 // by the key producer, launch_morton or launch_route_keys).
 hipError_t launch_sort(const Segment* segs, int64_t S, int64_t tiles_bound, SortBits bits,
