@@ -348,7 +348,15 @@ __global__ __launch_bounds__(kWave) void knn_tail_kernel(KnnArgs a, int groups) 
     const int slot = static_cast<int>(blockIdx.x) % kWave;
     for (int first = static_cast<int>(blockIdx.x) / kWave; first < groups; first += stride * kWave) {
         const int g = first + lane_id() * stride;
-        const uint64_t mask = g < groups ? a.tail_masks[g] : 0;
+        // The traversal wrote the marks of the work-groups that had queries:
+        // in a fallback few, those whose chunk starts inside its sub-list.
+        bool marked = g < groups;
+        if (a.fb_list != nullptr) {
+            const int r = g / kXcds;
+            const int sub = g % kXcds * kGridSubLists + r % kGridSubLists;
+            marked = marked && static_cast<uint32_t>(r / kGridSubLists * kKnnBlock) < a.fb_count[sub * kCountStride];
+        }
+        const uint64_t mask = marked ? a.tail_masks[g] : 0;
         uint64_t todo = __ballot((mask >> slot) & 1ull);
         while (todo != 0) {
             const int block = first + __builtin_ctzll(todo) * stride;
