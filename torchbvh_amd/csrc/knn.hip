@@ -793,6 +793,10 @@ __device__ __forceinline__ void knn_query(const KnnArgs& a) {
     int64_t gid = tile * kKnnBlock + threadIdx.x;
     float seed = kFar;
     if (fallback) {
+        for (int64_t i = static_cast<int64_t>(blockIdx.x) * kKnnBlock + threadIdx.x; i < a.fb_nflags;
+             i += static_cast<int64_t>(gridDim.x) * kKnnBlock) {
+            a.fb_flags[i] = 0u;
+        }
         const int64_t listed = a.fb_count[grid_sublist() * kCountStride];
         const int64_t at = grid_chunk_start() + threadIdx.x;
         gid = a.total_q;
@@ -932,13 +936,14 @@ __device__ __forceinline__ void grid_cell(const float* p, const float* lo, const
 // with probability below 1e-14).
 constexpr int kGridMaxGap = 64;
 
-// Clears the clouds' flags and the failure lists' counts (`ncounts` of
-// them, kCountStride words apart).
-__global__ void grid_init_kernel(uint32_t* flags, int64_t B, uint32_t* counts, int ncounts) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < B) flags[i] = 0u;
-    if (i < ncounts) counts[i * kCountStride] = 0u;
-}
+// A cloud's flag in the (uncleared) workspace: any other value enables it.  A
+// value left over from elsewhere that happens to be this one only sends the
+// cloud's queries to the traversal, whose results are the same; the fallback,
+// the search's last reader of the workspace's lists, clears the flags, so a
+// later call in the same memory, or a replay, does not meet this one's.
+// (Clearing them first was a launch of its own, 2 to 5 us: builds and calls of
+// 4M planar queries, k = 8 1126 -> 1117 us, 1M 3-D ones, k = 16 495 -> 491.)
+constexpr uint32_t kCloudDisabled = 0x9d15ab1eu;
 
 // Appends the lanes set in `left` (wave-uniform) to this work-group's
 // sub-list of a failure list (`seg` entries each).  A sub-list holds the
@@ -965,7 +970,7 @@ __device__ __forceinline__ void grid_append(int32_t* list, uint32_t* counts, int
 
 // One thread per point: writes the first-point entries of the cells from the
 // previous point's cell (exclusive) to its own, and after the last point
-// those up to the end.  flags[b] = 1 disables cloud b: a non-finite point or
+// those up to the end.  flags[b] = kCloudDisabled disables cloud b: a non-finite point or
 // box, an empty extent, a cell order that does not follow the points' (the
 // box is not the one their codes were taken against), or an empty run
 // longer than kGridMaxGap (its entries are then left unwritten, and unread).
@@ -984,7 +989,11 @@ struct GridTable {
 };
 template <int D>
 __global__ __launch_bounds__(kBlock) void grid_table_kernel(GridTable first, GridTable second, unsigned first_groups,
-                                                            int64_t B) {
+                                                            int64_t B, uint32_t* __restrict__ counts) {
+    // The failure lists' counts, for the passes that follow.
+    if (blockIdx.x == 0) {
+        for (int i = threadIdx.x; i < 2 * kGridCounts; i += kBlock) counts[i * kCountStride] = 0u;
+    }
     const bool is_second = blockIdx.x >= first_groups;
     const GridTable g = is_second ? second : first;
     const float4* __restrict__ pts = g.pts;
@@ -1034,7 +1043,7 @@ __global__ __launch_bounds__(kBlock) void grid_table_kernel(GridTable first, Gri
     }
     const int64_t last = j == n - 1 ? cells : own;  // after the last point: every cell to the end
     if (!ok || own < prev || own - prev > kGridMaxGap || last - own > kGridMaxGap) {
-        flags[b] = 1u;
+        flags[b] = kCloudDisabled;
         return;
     }
     for (int64_t c = prev + 1; c <= own; ++c) t[c] = j;
@@ -1222,14 +1231,14 @@ __global__ __launch_bounds__(kKnnBlock) void grid_knn_kernel(KnnArgs a, const fl
             in = locate<true, false, true, true>(a, gid);
             valid = in.row >= 0;
         }
-        ok = valid && flags[(in.second ? a.B : 0) + b] == 0u;
+        ok = valid && flags[(in.second ? a.B : 0) + b] != kCloudDisabled;
         if (__ballot(ok) == 0) {
             grid_append(list, counts, seg, __ballot(launched), gid);
             if (launched) bounds[gid] = kFar;
             return;
         }
     } else {
-        ok = valid && flags[b] == 0u;
+        ok = valid && flags[b] != kCloudDisabled;
         if (__ballot(ok) == 0) {
             grid_append(list, counts, seg, __ballot(valid), gid);
             if (valid) bounds[gid] = kFar;
@@ -1829,11 +1838,13 @@ void launch_grid_dk(const KnnArgs& a, int pass, const float* node_aabbs, int64_t
 
 // `second` with null points: none.
 template <int D>
-void launch_grid_table(const GridTable& first, const GridTable& second, int64_t B, hipStream_t stream) {
+void launch_grid_table(const GridTable& first, const GridTable& second, int64_t B, uint32_t* counts,
+                       hipStream_t stream) {
     auto groups = [&](const GridTable& g) {
         return g.pts ? static_cast<unsigned>((B * static_cast<int64_t>(g.n) + kBlock - 1) / kBlock) : 0u;
     };
-    grid_table_kernel<D><<<groups(first) + groups(second), kBlock, 0, stream>>>(first, second, groups(first), B);
+    grid_table_kernel<D><<<groups(first) + groups(second), kBlock, 0, stream>>>(first, second, groups(first), B,
+                                                                                      counts);
 }
 }  // namespace
 
@@ -1863,10 +1874,6 @@ hipError_t launch_grid_knn(const KnnArgs& args, const float* node_aabbs, int64_t
     int32_t* list2 = reinterpret_cast<int32_t*>(base + g.list2);
     float* bounds = reinterpret_cast<float*>(base + g.bounds);
     const GridSecond g2{node_aabbs2, nr2, level2, reinterpret_cast<const int32_t*>(base + g.table2)};
-    const int64_t nflags = args.B * (routed ? 2 : 1);
-    const int64_t init = std::max<int64_t>(nflags, 2 * kGridCounts);
-    grid_init_kernel<<<static_cast<unsigned>((init + kBlock - 1) / kBlock), kBlock, 0, stream>>>(flags, nflags, counts,
-                                                                                                2 * kGridCounts);
     const GridTable first{static_cast<const float4*>(args.accel), node_aabbs, nr, static_cast<int>(args.num_leaves),
                           level, table, flags};
     GridTable second{};
@@ -1875,8 +1882,8 @@ hipError_t launch_grid_knn(const KnnArgs& args, const float* node_aabbs, int64_t
                            static_cast<int>(args.num_leaves2), level2,
                            reinterpret_cast<int32_t*>(base + g.table2), flags + args.B};
     }
-    if (D == 3) launch_grid_table<3>(first, second, args.B, stream);
-    else launch_grid_table<2>(first, second, args.B, stream);
+    if (D == 3) launch_grid_table<3>(first, second, args.B, counts, stream);
+    else launch_grid_table<2>(first, second, args.B, counts, stream);
     const int passes = grid_second_pass(D, K) ? 2 : 1;
     for (int pass = 1; pass <= passes; ++pass) {
         auto run = [&](auto dk) {
@@ -1912,6 +1919,8 @@ hipError_t launch_grid_knn(const KnnArgs& args, const float* node_aabbs, int64_t
     f.fb_bound = bounds;
     f.fb_count = passes == 2 ? counts2 : counts;
     f.fb_seg = g.seg;
+    f.fb_flags = flags;
+    f.fb_nflags = args.B * (routed ? 2 : 1);
     if (tail_workspace_bytes(args.total_q, D) == 0) return launch_knn_accel(f, D, K, false, stream);
     // The queries it gives up: masks in the list that is not in use (a
     // work-group's 64 entries of it hold its mask), bounds in place.

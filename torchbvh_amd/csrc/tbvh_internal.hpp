@@ -474,6 +474,9 @@ struct KnnArgs {
     const float* fb_bound;
     const uint32_t* fb_count;
     int64_t fb_seg;
+    // The search's cloud flags, which the fallback clears.
+    uint32_t* fb_flags;
+    int64_t fb_nflags;
     // Tail (accel only; null: none): queries that a traversal wave gives up
     // (see traverse) are marked in tail_masks[work-group], bit per lane, with
     // their k-th distance so far in tail_bounds[launch position], and
