@@ -94,10 +94,13 @@ __device__ __forceinline__ uint64_t reversed64(uint64_t k) {
     return (lane_id() & 32) ? even : odd;
 }
 
-// key_max with a wave-uniform second operand.
+// key_max with a wave-uniform second operand.  A vector instruction may read a
+// scalar register only two wait states after another vector instruction (the
+// v_readlane that `add` has the key from) wrote it; the compiler inserts them
+// for its own instructions and not for those in inline assembly.
 __device__ __forceinline__ uint64_t key_max_uniform(uint64_t a, uint64_t b) {
     double r;
-    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(__longlong_as_double(a)), "s"(__longlong_as_double(b)));
+    asm("s_nop 1\n\tv_max_f64 %0, %1, %2" : "=v"(r) : "v"(__longlong_as_double(a)), "s"(__longlong_as_double(b)));
     return static_cast<uint64_t>(__double_as_longlong(r));
 }
 
