@@ -180,3 +180,32 @@ def test_given_up_routed_queries(dim, k):
                                                     payload["num_leaves"], payload["num_real_nodes"], dim, k)
         assert torch.equal(i[0, sel], ei[0] + offset)
         assert torch.equal(d2[0, sel], ed[0])
+
+
+@pytest.mark.parametrize("layout", ["batched", "ragged"])
+@pytest.mark.parametrize("k", [16, 32])
+def test_given_up_queries_among_nan_points(layout, k):
+    """Points with a NaN coordinate are near on their other axes, in boxes that
+    are not.  Here the traversal scans one eighth first, 16 near points and 15
+    with a NaN y beside one far in y, gives the query up over the shell in the
+    other eighths, and the boxes within its k-th distance hold fewer than k
+    points: the rows must still be distinct points at their true distances."""
+    rng = np.random.default_rng(1)
+    v = rng.standard_normal((3000, 3))
+    v = v / np.linalg.norm(v, axis=1, keepdims=True) * (1 + 1e-3 * rng.random((3000, 1)))
+    nan = np.stack([-0.05 - 0.4 * rng.random(15), np.full(15, np.nan), -0.05 - 0.4 * rng.random(15)], 1)
+    near = np.stack([-5e-4 - 0.05 * rng.random(16), -5e-4 - 0.05 * rng.random(16), -0.99 - 1e-4 * rng.random(16)], 1)
+    near[0, :2] = -5e-4
+    pts = np.concatenate([v[~(v < 0).all(1)], nan, [[-0.25, -1.0, -0.25]], near]).astype(np.float32)
+    q = (-2e-3 + 5e-4 * rng.standard_normal((30_000, 3))).astype(np.float32)
+    tp, tq = torch.from_numpy(pts).cuda(), torch.from_numpy(q).cuda()
+    if layout == "ragged":
+        offsets = torch.tensor([0, len(pts)], device="cuda"), torch.tensor([0, len(q)], device="cuda")
+        idx, d2 = tb.query_knn(tb.build_bvh(tp, batch_offsets=offsets[0]), tq, k, query_offsets=offsets[1])
+    else:
+        idx, d2 = tb.query_knn(tb.build_bvh(tp), tq, k)
+    idx, d2 = idx.cpu().numpy(), d2.cpu().numpy()
+    assert (idx >= 0).all()
+    assert (np.diff(np.sort(idx, axis=1), axis=1) > 0).all()
+    assert (np.diff(d2, axis=1) >= 0).all()
+    assert np.array_equal(d2, oracle.pair_distances(pts, q, idx))

@@ -184,8 +184,12 @@ struct WaveQuery {
         L = tree::leaf_level(n);
         vl = tree::virtual_leaves(n);
         bl = L > kBlockBits ? L - kBlockBits : 0;
+        restart(bound);
+    }
+
+    // Entries (bound, -1) in every lane: K points displace those below K.
+    __device__ __forceinline__ void restart(float bound) {
         filled = false;
-        // Entries (bound, -1) in every lane: K points displace those below K.
         list = candidate_key(bound, 0xffffffffu);
         kth = list;
         worst = bound;
@@ -320,11 +324,19 @@ __device__ __forceinline__ void wave_search(const KnnArgs& a, const QueryLoc& l,
            static_cast<const float4*>(l.second ? a.accel2 : a.accel) + l.pstart, l.n, bound);
 #pragma unroll
     for (int d = 0; d < D; ++d) w.q[d] = a.queries[l.row * D + d];
-    switch (kSteps > 0 ? kSteps : wave_steps(l.n)) {
-        case 1: w.template expand<0>(0); break;
-        case 2: w.template expand<1>(0); break;
-        case 3: w.template expand<2>(0); break;
-        default: w.template expand<3>(0); break;
+    // A second time, without the bound, when it kept out points that it stands
+    // for: the boxes do not bound the distance of a point with a NaN
+    // coordinate, which the traversal may have reached on another way.
+    while (true) {
+        switch (kSteps > 0 ? kSteps : wave_steps(l.n)) {
+            case 1: w.template expand<0>(0); break;
+            case 2: w.template expand<1>(0); break;
+            case 3: w.template expand<2>(0); break;
+            default: w.template expand<3>(0); break;
+        }
+        if (!(bound < kFar) || static_cast<uint32_t>(w.kth) != 0xffffffffu) break;
+        bound = kFar;
+        w.restart(bound);
     }
     write_list<D, K>(a, w.list, l.out_row, l.index_offset, l.pstart);
 }
