@@ -110,3 +110,30 @@ def test_binding_indices_out_of_range_add_nothing():
     got = _C.interpolate_neighbors_backward(up, idx, w, none)
     valid = (idx >= 0) & (idx < 10)
     assert torch.equal(got, _C.interpolate_neighbors_backward(up, idx.clamp(0, 9), w * valid, none))
+
+
+@pytest.mark.parametrize("how", ["batched", "vmap", "tangent", "around"])
+def test_backward_under_transforms(monkeypatch, how):
+    """The forward ran in the kernels; the backward meets transforms that they
+    can't take (and the forward itself, one around plain values)."""
+    pos, q, values, up = _inputs(1, 64, 2, 3, 3, 6)
+    ups = torch.randn((3, *up.shape), generator=torch.Generator("cuda").manual_seed(7), device="cuda")
+
+    def compute():
+        v = values.clone().requires_grad_()
+        if how == "around":
+            f = lambda s: (s * tb.interpolate_displaced(pos, q, v, 4) * up).sum()  # noqa: E731
+            return torch.autograd.grad(torch.func.vmap(f)(torch.ones(2, device="cuda")).sum(), v)[0]
+        out = tb.interpolate_displaced(pos, q, v, 4)
+        if how == "batched":
+            return torch.autograd.grad(out, v, ups, is_grads_batched=True)[0]
+        if how == "vmap":
+            return torch.func.vmap(lambda u: torch.autograd.grad(out, v, u, retain_graph=True)[0])(ups)
+        with torch.autograd.forward_ad.dual_level():
+            g = torch.autograd.grad(out, v, torch.autograd.forward_ad.make_dual(ups[0], ups[1]))[0]
+            return torch.stack(tuple(torch.autograd.forward_ad.unpack_dual(g)))
+
+    got = compute()
+    monkeypatch.setattr(_multihead, "_kernels_differentiate", lambda *a: False)
+    # Sums of up to 64 terms of size about one, in another order.
+    torch.testing.assert_close(got, compute(), rtol=0, atol=64 * 2.0**-22)

@@ -93,15 +93,50 @@ def gather_neighbor_values(values: torch.Tensor, indices: torch.Tensor) -> torch
         lo, hi = torch.aminmax(indices)
         if int(lo) < 0 or int(hi) >= values.size(1):
             raise ValueError(_NOT_LOCAL)
+    return _gather(values, indices)
+
+
+def _gather(values: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
     B, _, H, _ = values.shape
     batch = torch.arange(B, device=values.device).view(B, 1, 1, 1)
     head = torch.arange(H, device=values.device).view(1, 1, H, 1)
     return values[batch, indices, head]
 
 
+def _combine(neighbours: torch.Tensor, weights: torch.Tensor, exact: torch.Tensor) -> torch.Tensor:
+    """(B, N, H, k, Ch) neighbours to their weighted means, or those of a row's
+    exact hits.  Accumulated neighbour rank by neighbour rank, the reference's
+    order of fp32 additions (_multihead.py:123-144)."""
+    weighted = torch.zeros_like(neighbours[..., 0, :])
+    exact_sum = torch.zeros_like(weighted)
+    for r in range(neighbours.size(-2)):
+        v = neighbours[..., r, :]
+        weighted = weighted + v * weights[..., r].unsqueeze(-1)
+        exact_sum = exact_sum + v * exact[..., r].to(neighbours.dtype).unsqueeze(-1)
+    if exact.any():
+        counts = exact.to(neighbours.dtype).sum(dim=-1, keepdim=True).clamp(min=1.0)
+        weighted = torch.where(exact.any(dim=-1, keepdim=True), exact_sum / counts, weighted)
+    return weighted
+
+
+def _spread(grad: torch.Tensor, indices: torch.Tensor, weights: torch.Tensor, exact: torch.Tensor) -> torch.Tensor:
+    """The transpose of `_combine` of `_gather` by tensor operations."""
+    B, N, H, C = grad.shape
+    hit = exact.to(grad.dtype)
+    mean = grad / hit.sum(dim=-1, keepdim=True).clamp(min=1.0)
+    parts = torch.where(exact.any(dim=-1, keepdim=True).unsqueeze(-1), mean.unsqueeze(-2) * hit.unsqueeze(-1),
+                        grad.unsqueeze(-2) * weights.unsqueeze(-1))
+    batch = torch.arange(B, device=grad.device).view(B, 1, 1, 1)
+    head = torch.arange(H, device=grad.device).view(1, 1, H, 1)
+    rows = ((batch * N + indices) * H + head).reshape(-1)
+    zeros = torch.zeros((B * N * H, C), dtype=grad.dtype, device=grad.device)
+    return zeros.index_put((rows,), parts.reshape(-1, C), accumulate=True).reshape(B, N, H, C)
+
+
 class _Interpolate(torch.autograd.Function):
     """`_C.interpolate_neighbors`, differentiable (any number of times) in its
-    values: the result is linear in them."""
+    values: the result is linear in them.  The backward may run under other
+    transforms than the forward did, so it chooses again."""
 
     @staticmethod
     def forward(values, indices, weights, exact):
@@ -113,7 +148,8 @@ class _Interpolate(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):
-        return _InterpolateTransposed.apply(grad, *ctx.saved_tensors), None, None, None
+        linear = _InterpolateTransposed.apply if _is_plain(grad) else _spread
+        return linear(grad, *ctx.saved_tensors), None, None, None
 
 
 class _InterpolateTransposed(torch.autograd.Function):
@@ -129,21 +165,32 @@ class _InterpolateTransposed(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):
-        return _Interpolate.apply(grad, *ctx.saved_tensors), None, None, None
+        indices, weights, exact = ctx.saved_tensors
+        if _is_plain(grad):
+            return _Interpolate.apply(grad, indices, weights, exact), None, None, None
+        return _combine(_gather(grad, indices), weights, exact), None, None, None
+
+
+def _is_plain(tensor: torch.Tensor) -> bool:
+    """Whether the library's kernels may take `tensor` in an autograd function:
+    its memory holds its values, and no transform has to see the tensor
+    operations (functorch levels, which also refuse such functions around
+    tensors they don't wrap, batched gradients, forward-mode, dispatch and
+    function modes, tracing)."""
+    C = torch._C
+    return (type(tensor) in (torch.Tensor, torch.nn.Parameter)
+            and not C._are_functorch_transforms_active()
+            and not C._functorch.is_legacy_batchedtensor(tensor)
+            and not tensor.is_neg() and not tensor._is_zerotensor()
+            and torch.autograd.forward_ad._current_level < 0
+            and C._len_torch_dispatch_stack() == 0 and C._len_torch_function_stack() == 0
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 
 def _kernels_differentiate(values: torch.Tensor, indices: torch.Tensor) -> bool:
     """Whether the differentiable call may run as the library's kernels: plain
-    tensors outside of every transform that has to see the tensor operations
-    (functorch levels, forward-mode, dispatch and function modes, tracing),
-    and entry counts the backward's sort can number."""
-    C = torch._C
-    return (type(values) in (torch.Tensor, torch.nn.Parameter)
-            and not C._functorch.is_functorch_wrapped_tensor(values)
-            and torch.autograd.forward_ad._current_level < 0
-            and C._len_torch_dispatch_stack() == 0 and C._len_torch_function_stack() == 0
-            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
-            and 0 < indices.numel() <= 2**31 - 1)
+    values, and entry counts the backward's sort can number."""
+    return _is_plain(values) and 0 < indices.numel() <= 2**31 - 1
 
 
 def interpolate_displaced(pos: torch.Tensor, q: torch.Tensor, values: torch.Tensor, k: int = 8, *,
@@ -191,16 +238,4 @@ def interpolate_displaced(pos: torch.Tensor, q: torch.Tensor, values: torch.Tens
         if int(least) < 0:
             raise ValueError(_NOT_LOCAL)
         return out
-    neighbours = gather_neighbor_values(values, indices)  # (B, N, H, k, Ch)
-    # Accumulated neighbour rank by neighbour rank, the reference's order of
-    # fp32 additions (_multihead.py:123-144).
-    weighted = torch.zeros_like(values)
-    exact_sum = torch.zeros_like(values)
-    for r in range(indices.size(-1)):
-        v = neighbours[..., r, :]
-        weighted = weighted + v * weights[..., r].unsqueeze(-1)
-        exact_sum = exact_sum + v * exact[..., r].to(values.dtype).unsqueeze(-1)
-    if exact.any():
-        counts = exact.to(values.dtype).sum(dim=-1, keepdim=True).clamp(min=1.0)
-        weighted = torch.where(exact.any(dim=-1, keepdim=True), exact_sum / counts, weighted)
-    return weighted
+    return _combine(gather_neighbor_values(values, indices), weights, exact)
