@@ -1,7 +1,8 @@
 """Properties of the compiled device code that no run shows reliably: the wait
-states between dependent vector instructions.  The compiler keeps them for its
-own instructions, not for those written as inline assembly, which it schedules
-without looking inside."""
+states between dependent vector instructions, which the compiler keeps for its
+own instructions but not for those written as inline assembly (it schedules
+without looking inside), and the registers that the traversals are written to
+fit in."""
 import functools
 import os
 import re
@@ -149,3 +150,32 @@ def test_checker_finds_a_missing_wait():
 def test_wait_states_between_dependent_vector_instructions(assembly, source):
     missing = [m for body in _kernels(assembly[source]) for m in _missing_waits(body)]
     assert not missing, f"{len(missing)} sites, e.g. {missing[:3]}"
+
+
+def _vector_registers(assembly: str, kernel: str) -> dict:
+    """{template arguments: allocated VGPRs} of the kernels of that name."""
+    found = {}
+    for name, body in re.findall(r"\.amdhsa_kernel (\S+)\n(.*?)\.end_amdhsa_kernel", assembly, re.S):
+        arguments = re.search(rf"\d{kernel}I((?:L[ib]\d+E)+)E", name)
+        if arguments:
+            key = tuple(int(x) for x in re.findall(r"L[ib](\d+)E", arguments.group(1)))
+            found[key] = int(re.search(r"\.amdhsa_next_free_vgpr (\d+)", body).group(1))
+    return found
+
+
+# Waves per SIMD (512 registers in all, allocated in eights).
+@pytest.mark.parametrize("dim,k,waves", [(2, 4, 7), (2, 8, 8), (2, 16, 4), (2, 32, 4),
+                                         (3, 4, 7), (3, 8, 7), (3, 16, 4), (3, 32, 3)])
+def test_implicit_tree_traversal_keeps_its_occupancy(assembly, dim, k, waves):
+    registers = _vector_registers(assembly["knn.hip"], "knn_kernel")
+    for ordered in (0, 1):  # (D, K, ordered, ragged, routed)
+        used = registers[(dim, k, ordered, 0, 0)]
+        assert 512 // (-(-used // 8) * 8) >= waves, used
+
+
+@pytest.mark.parametrize("dim,k,compact,waves", [(2, 8, 0, 8), (3, 8, 0, 7), (3, 16, 0, 6), (3, 16, 1, 6), (3, 32, 0, 4)])
+def test_accel_traversal_keeps_its_occupancy(assembly, dim, k, compact, waves):
+    registers = _vector_registers(assembly["knn.hip"], "knn_accel_kernel")
+    for ordered in (0, 1):  # (D, K, ordered, ragged, routed, compact)
+        used = registers[(dim, k, ordered, 0, 0, compact)]
+        assert 512 // (-(-used // 8) * 8) >= waves, used

@@ -799,23 +799,16 @@ __device__ __forceinline__ void knn_query(const KnnArgs& a) {
         }
         const int64_t listed = a.fb_count[grid_sublist() * kCountStride];
         const int64_t at = grid_chunk_start() + threadIdx.x;
-        gid = a.total_q;
-        if (at < listed) {
-            gid = a.fb_list[grid_sublist() * a.fb_seg + at];
-            seed = a.fb_bound[gid];
-        }
+        if (at >= listed) return;
+        gid = a.fb_list[grid_sublist() * a.fb_seg + at];
+        seed = a.fb_bound[gid];
     }
-    QueryLoc in{};
-    in.row = -1;
-    if (gid < a.total_q) in = locate<kOrdered, kRagged, kRouted, kAccel>(a, gid);
-    const bool tail = kAccel && a.tail_masks != nullptr;
-    if (__ballot(in.row >= 0) == 0) {
-        // (A fallback's work-group past its sub-list's end has no mask: the
-        // tail does not read it.)
-        if (tail && threadIdx.x == 0 && (!fallback || gid < a.total_q)) a.tail_masks[blockIdx.x] = 0;
-        return;
-    }
+    // A work-group that ends here writes no mask for the tail: it has no
+    // positions, or no rows at any (the tail looks for both again).
+    if (gid >= a.total_q) return;
+    const QueryLoc in = locate<kOrdered, kRagged, kRouted, kAccel>(a, gid);
     if (in.row < 0) return;
+    const bool tail = kAccel && a.tail_masks != nullptr;
 
     float q[D];
 #pragma unroll

@@ -363,13 +363,18 @@ __global__ __launch_bounds__(kWave) void knn_tail_kernel(KnnArgs a, int groups) 
     const int slot = static_cast<int>(blockIdx.x) % kWave;
     for (int first = static_cast<int>(blockIdx.x) / kWave; first < groups; first += stride * kWave) {
         const int g = first + lane_id() * stride;
-        // The traversal wrote the marks of the work-groups that had queries:
-        // in a fallback few, those whose chunk starts inside its sub-list.
+        // The traversal wrote the marks of the work-groups that had queries;
+        // this one looks at positions inside the call or, in a fallback,
+        // inside their sub-list (few work-groups have any).
+        const int r = g / kXcds;
         bool marked = g < groups;
         if (a.fb_list != nullptr) {
-            const int r = g / kXcds;
             const int sub = g % kXcds * kGridSubLists + r % kGridSubLists;
-            marked = marked && static_cast<uint32_t>(r / kGridSubLists * kKnnBlock) < a.fb_count[sub * kCountStride];
+            const int64_t at = static_cast<int64_t>(r / kGridSubLists) * kKnnBlock + slot;
+            marked = marked && at < a.fb_count[sub * kCountStride];
+        } else {
+            const int64_t tile = static_cast<int64_t>(g % kXcds) * (groups / kXcds) + r;
+            marked = marked && tile * kKnnBlock + slot < a.total_q;
         }
         const uint64_t mask = marked ? a.tail_masks[g] : 0;
         uint64_t todo = __ballot((mask >> slot) & 1ull);
