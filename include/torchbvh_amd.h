@@ -202,7 +202,7 @@ int tbvh_sort_queries_ragged(const float* queries, const int64_t* query_offsets,
 /* The schedule of a search for k neighbours (the other arguments and the workspace as for
  * the sorts above): `order` [B, M] or [total_q], local query indices per cloud, in
  * nearly the order of the top 24 bits of the queries' Hilbert (k = 32) or Morton
- * index; calls need not repeat it. */
+ * index, the same on every call. */
 int tbvh_schedule_queries_fine(const float* queries, int64_t B, int64_t M, int D, int k,
                                const float* scene_min, const float* scene_max,
                                int64_t* order,

@@ -34,6 +34,8 @@ def test_order(B, M, dim, kind):
     for k in (8, 32):  # Morton, Hilbert
         order = _C.morton_sort_queries_narrow(q, lo, hi, schedule=True, fine=k)
         assert torch.equal(order.sort(1)[0], torch.arange(M, device="cuda").expand(B, M))
+        for _ in range(3):  # every call gives the same
+            assert torch.equal(order, _C.morton_sort_queries_narrow(q, lo, hi, schedule=True, fine=k))
         if k == 8:
             bits = 30 if dim == 3 else 32
             codes = _C.morton_codes(q, lo, hi).gather(1, order)

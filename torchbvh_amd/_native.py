@@ -786,8 +786,8 @@ class _NativeOps:
                                    fine: int | None = None) -> torch.Tensor:
         """Stable Morton order of [B, M, D] queries against per-cloud bounds.
         With ``schedule`` the order of the top 16 bits of Hilbert keys instead;
-        with ``fine`` = k too, the schedule ``query_knn`` uses, nearly the order of
-        24 bits and not the same on every call (results do not depend on it)."""
+        with ``fine`` = k too, nearly the order of 24 bits (results do not depend
+        on it)."""
         op = "morton_sort_queries_narrow"
         _require_device_f32(op, queries, "queries")
         _require(scene_min.is_cuda and scene_max.is_cuda and scene_min.is_contiguous()

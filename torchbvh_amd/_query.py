@@ -170,9 +170,12 @@ SCHEDULE_MIN_QUERIES = 1 << 17
 
 
 # From this many queries per cloud the schedule also orders the queries inside
-# a cell of its 16-bit keys (16 of them at a million).  Ordering and search of
-# uniform clouds, us, without / with: 2-D 4M k = 8 730 / 694, 3-D 1M k = 16 336 / 322;
-# 300,000 k = 8 213 / 222.
+# a cell of its 16-bit keys (16 of them at a million).  Ordering and search, us,
+# without / with.  Uniform 3-D k = 16: 524,288 278 / 284, 917,504 541 / 545, 1,048,576
+# 310 / 309, 2M 646 / 628; k = 8: 163 / 167, 215 / 215, 240 / 236, 544 / 491; 2-D k = 8: 136 / 144,
+# 204 / 211, 219 / 218, 409 / 372; 3-D k = 32: 420 / 431, 880 / 887, 914 / 919, 1046 / 1033.
+# Eight clusters, k = 16: 262,144 246 / 260, 524,288 467 / 459, 1,048,576 847 / 771; a surface
+# 174 / 179, 302 / 297, 499 / 482.
 FINE_MIN_QUERIES = 1 << 20
 
 

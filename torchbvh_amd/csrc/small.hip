@@ -340,11 +340,17 @@ void launch_d(const float* rows, const Segment* segs, int64_t S, UniformPlan pla
 }
 
 // The rows of one sort tile, already in order of their keys' top 16 bits, into
-// order of all their bits (nearly: rows of one slot stay in any order), for a
-// schedule, whose order changes no result.  Bins over the tile's key range and sub-bins as in
-// the small sort, by the key's place in the range.  One read and one write of 8
-// bytes a row: 9 us at 1M rows, 20 at 4M, where two more passes of the global sort
-// took 32 and 66.
+// order of all their bits (nearly), for a schedule, whose order changes no
+// result.  Bins over the tile's key range and sub-bins as in the small sort, by
+// the key's place in the range.  One read and one write of 8 bytes a row: 8 us at
+// 1M rows, 24 at 4M, where two more passes of the global sort took 32 and 66.
+//
+// Every call gives the same order: among points with a NaN coordinate a search's
+// rows depend on which queries share a wave.  Rows of a slot in the order they
+// reach it, which differs from call to call, took 6 and 13 us.  A tile with more than
+// kMostInBin rows in a slot stays as it is (1M points and queries, k = 16, ordering
+// and search with that limit 32 / 128 / none, us: 8 clusters 758 / 763 / 940, 500 tight ones
+// 1208 / 1163 / 1290, 40 copies of each point 309 / 318 / 317).
 __global__ __launch_bounds__(kSmallThreads) void refine_kernel(const Segment* __restrict__ segs, int S, int key_bits,
                                                                const uint32_t* __restrict__ keys,
                                                                const uint32_t* __restrict__ vals,
@@ -396,10 +402,40 @@ __global__ __launch_bounds__(kSmallThreads) void refine_kernel(const Segment* __
             at[i] = slot | count_half(sub, slot) << 16;
         }
     }
-    scan_halves<kItems>(sub, s_scan);
+    // Rows of one slot keep their order in the tile: their arrivals, which
+    // differ from call to call, are ranked by it.
+    uint32_t most = 0;
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
-        if (i * kSmallThreads + threadIdx.x < count) s_vals[read_half(sub, at[i] & 0xffffu) + (at[i] >> 16)] = val[i];
+        if (i * kSmallThreads + threadIdx.x < count) most = max(most, at[i] >> 16);
+    }
+    if (__syncthreads_or(most >= kMostInBin)) {
+        // Many rows of one key or nearly: the tile stays as it is.
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            const int j = i * kSmallThreads + threadIdx.x;
+            if (j < count) order[row0 + j] = static_cast<int64_t>(val[i]);
+        }
+        return;
+    }
+    scan_halves<kItems>(sub, s_scan);
+    uint16_t* arrivals = reinterpret_cast<uint16_t*>(bins);
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        const int j = i * kSmallThreads + threadIdx.x;
+        if (j < count) arrivals[read_half(sub, at[i] & 0xffffu) + (at[i] >> 16)] = static_cast<uint16_t>(j);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        const int j = i * kSmallThreads + threadIdx.x;
+        if (j < count) {
+            const uint32_t slot = at[i] & 0xffffu;
+            const uint32_t first = read_half(sub, slot), end = read_half(sub, slot + 1);
+            uint32_t place = first;
+            for (uint32_t o = first; o < end; ++o) place += arrivals[o] < j ? 1u : 0u;
+            s_vals[place] = val[i];
+        }
     }
     __syncthreads();
     for (int j = threadIdx.x; j < count; j += kSmallThreads) order[row0 + j] = static_cast<int64_t>(s_vals[j]);
