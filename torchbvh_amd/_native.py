@@ -274,7 +274,12 @@ GRID_MIN_QUERIES = 1 << 17
 # queries k = 4 90 / 104, 32,000 137 / 119.  2-D boxes overlap less, so the
 # traversal is shorter: 10,000 points, 16,000 queries k = 4 32 / 34; 50,000 points,
 # 8,000 queries k = 4 30 / 39, 16,000 45 / 39; 300,000 points, 4,000 queries k = 4
-# 40 / 44, 8,000 57 / 43, k = 8 57 / 64.
+# 40 / 44, 8,000 57 / 43, k = 8 57 / 64.  Queries near a circle lose by it, queries far
+# from one would lose more without (2-D, k = 4 and 16): 20,000 points, 10,000 queries
+# 43 / 27 and 45 / 36; 150,000 points, 1,000 queries 45 / 28 and 50 / 41, 6,000 65 / 29
+# and 72 / 44; far from it, 300,000 points, 1,000 queries k = 16 150 / 3540, 4,000 231 / 5000.
+# Near the limit on large 3-D clouds too: 500,000 points of a sphere, 20,000 queries
+# 1.08 times the traversal's time, of a lattice of 4,913 sites 1.4 times; far 1,400 / 18,000.
 WAVE_MAX_QUERIES = 24 << 10         # 3-D
 WAVE_MAX_QUERIES_2D = 12 << 10      # 2-D, clouds of at most WAVE_2D_CLOUD points
 WAVE_MAX_QUERIES_2D_LARGE = 6 << 10
