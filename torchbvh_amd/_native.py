@@ -277,9 +277,9 @@ GRID_MIN_QUERIES = 1 << 17
 # 40 / 44, 8,000 57 / 43, k = 8 57 / 64.  Queries near a circle lose by it, queries far
 # from one would lose more without (2-D, k = 4 and 16): 20,000 points, 10,000 queries
 # 43 / 27 and 45 / 36; 150,000 points, 1,000 queries 45 / 28 and 50 / 41, 6,000 65 / 29
-# and 72 / 44; far from it, 300,000 points, 1,000 queries k = 16 150 / 3540, 4,000 231 / 5000.
+# and 72 / 44; far from it, 300,000 points, k = 16, 1,000 queries 134 / 3510, 6,000 212 / 5690.
 # Near the limit on large 3-D clouds too: 500,000 points of a sphere, 20,000 queries
-# 1.08 times the traversal's time, of a lattice of 4,913 sites 1.4 times; far 1,400 / 18,000.
+# 1.08 times the traversal's time, of a lattice of 4,913 sites 1.4 times; far 1010 / 13280.
 WAVE_MAX_QUERIES = 24 << 10         # 3-D
 WAVE_MAX_QUERIES_2D = 12 << 10      # 2-D, clouds of at most WAVE_2D_CLOUD points
 WAVE_MAX_QUERIES_2D_LARGE = 6 << 10
