@@ -1,6 +1,6 @@
 """Benchmark: BVH build + exact k-NN on one MI355X.
 
-Default workload: 1,048,576 uniform 3-D points,
+Default workload (cfg2): 1,048,576 uniform 3-D points,
 1,048,576 uniform queries, k = 16, fp32.  One step = build the BVH, Morton-
 order the queries, run the traversal — the whole hot path, inputs resident in
 HBM.  Prints one JSON line.
@@ -11,7 +11,7 @@ HBM.  Prints one JSON line.
     python bench.py --extras      # spatial/routed k-NN, gather, primitive build, point order
     python bench.py --copy-floor  # plain device copies at the build kernels' byte counts
 
-The synthetic workloads of every BASELINE config are defined here
+The synthetic workloads of every config are defined here
 (``make_workload``) and shared with the parity tests.
 """
 
@@ -30,8 +30,8 @@ from pathlib import Path
 import torch
 
 # ---------------------------------------------------------------------------
-# Workloads (seeds and shapes as fixed for the BASELINE configs; generated on
-# the CPU so GPU, oracle and CPU baseline see bit-identical inputs)
+# Workloads (seeds and shapes are fixed; generated on the CPU so GPU, oracle
+# and CPU baseline see bit-identical inputs)
 # ---------------------------------------------------------------------------
 CONFIGS = {
     "cfg1": "3D k-NN, 10,000 uniform points / 10,000 uniform queries, k=4",
@@ -47,7 +47,7 @@ def _gen(seed: int) -> torch.Generator:
 
 
 def make_workload(name: str, scale: float = 1.0) -> dict:
-    """Return CPU tensors for a BASELINE config.
+    """Return CPU tensors for a config.
 
     ``scale`` < 1 shrinks the point/query counts (same distributions and
     seeds) for quick parity runs; 1.0 is the configured size.
@@ -123,10 +123,11 @@ def qsort_bytes(q: int, D: int) -> int:
     return q * (4 * D + 72)
 
 
-def qschedule_bytes(q: int, D: int) -> int:
+def qschedule_bytes(q: int, D: int, fine: bool = False) -> int:
     """The traversal schedule query_knn runs instead: the same terms with
-    two passes (the top 16 key bits) in place of four."""
-    return q * (4 * D + 40)
+    two passes (the top 16 key bits) in place of four; the fine one reads
+    keys and rows and writes the order once more."""
+    return q * (4 * D + (56 if fine else 40))
 
 
 def knn_bytes(q: int, D: int, k: int) -> int:
@@ -480,6 +481,50 @@ def copy_floor() -> int:
     return 0
 
 
+def query_phases(kind: str, bvh, queries, query_offsets, k: int, between):
+    """The binding calls of ``tb.query_knn`` (without its argument checks),
+    with `between` called after the ordering."""
+    from torchbvh_amd import _query
+    from torchbvh_amd._native import _C
+
+    dim = bvh["dim"]
+    if kind == "ragged":
+        clouds, total = bvh["batch_size"], int(queries.shape[0])
+        packed = bvh._aux["packed"]
+        offsets = _C.safe_offsets(query_offsets, total)
+        order = None
+        if _query._schedule(True, total):
+            order = _C.morton_sort_queries_ragged(queries, offsets, packed["scene_min"], packed["scene_max"], clouds,
+                                                  schedule=True)
+        between()
+        return _C.query_knn_ragged(
+            packed["node_aabbs"], packed["sorted_indices"], bvh["batch_offsets"], packed["node_offsets"],
+            queries, offsets, order, clouds, dim, k, accel=bvh._aux["accel"],
+            total_points=bvh._aux["host_offsets"][-1], source_points=None)
+    lead = (lambda t: t.unsqueeze(0)) if kind == "single" else (lambda t: t)
+    queries = lead(queries)
+    tree = (lead(bvh["node_aabbs"]), lead(bvh["sorted_indices"]), queries)
+    sizes = (bvh["num_leaves"], bvh["num_real_nodes"], dim, k)
+    accel = bvh._aux["accel"]
+    order = None
+    if _query._schedule(True, int(queries.shape[0] * queries.shape[1])):
+        order = _C.morton_sort_queries_narrow(queries, lead(bvh["scene_min"]), lead(bvh["scene_max"]), schedule=True,
+                                              **_query._fine(int(queries.shape[1]), k))
+    between()
+    if order is not None:
+        return _C.query_knn_batched_cached_bounds_ordered(*tree, order, *sizes, accel=accel, source_points=None)
+    return _C.query_knn_batched_cached_bounds(*tree, *sizes, accel=accel, source_points=None)
+
+
+def query_order(kind: str, clouds: int, total_q: int, k: int) -> str:
+    """Which order `query_phases` searches in: "input", "schedule" or "fine"."""
+    from torchbvh_amd import _query
+
+    if not _query._schedule(True, total_q):
+        return "input"
+    return "fine" if kind != "ragged" and _query._fine(total_q // clouds, k) else "schedule"
+
+
 def main() -> int:
     ap = argparse.ArgumentParser(description=__doc__)
     ap.add_argument("--gpus", type=int, default=1)
@@ -526,6 +571,7 @@ def main() -> int:
     qs = w["queries"].to(dev)
     D = pts.shape[-1]
     kind = w["kind"]
+    off = qoff = None
     if kind == "ragged":
         off = w["offsets"].to(dev)
         qoff = w["query_offsets"].to(dev)
@@ -538,23 +584,23 @@ def main() -> int:
     else:
         total_q = qs.shape[0]
         b_bytes = build_bytes(pts.shape[0], D)
-    s_bytes = qschedule_bytes(total_q, D)
+    order = query_order(kind, pts.shape[0] if kind == "batched" else 1, total_q, k)
+    order_what = {
+        "input": "none: at most SCHEDULE_MIN_QUERIES queries run in input order",
+        "schedule": "traversal schedule: stable 2-pass radix sort on the top 16 bits of Hilbert keys",
+        "fine": "traversal schedule: stable 2-pass radix sort on the top 16 bits of "
+                f"{'Hilbert' if k >= 32 else 'Morton'} keys, then their other bits within sort tiles",
+    }[order]
+    s_bytes = qschedule_bytes(total_q, D, order == "fine")
     full_sort_bytes = qsort_bytes(total_q, D)
     n_bytes = knn_bytes(total_q, D, k)
 
     from torchbvh_amd._native import _C
-    from torchbvh_amd._query import SCHEDULE_MIN_QUERIES
-
-    # query_knn schedules the traversal only above SCHEDULE_MIN_QUERIES
-    # queries (below it, input order is faster, schedule included).
-    scheduled = total_q > SCHEDULE_MIN_QUERIES
 
     def step(events=None):
         """One pass of the hot path: build (BVH + accel), query ordering,
-        traversal.  The build goes through the public API; the query calls
-        the native ops in the order ``tb.query_knn`` does, with an event
-        between each phase (all on torch's current stream, the stream the
-        kernels are launched on)."""
+        traversal, with an event between each phase (all on torch's current
+        stream, the stream the kernels are launched on)."""
         if events:
             events[0].record()
         if kind == "ragged":
@@ -563,35 +609,7 @@ def main() -> int:
             bvh = tb.build_bvh(pts)
         if events:
             events[1].record()
-        if kind == "ragged":
-            packed = bvh._aux["packed"]
-            order = (_C.morton_sort_queries_ragged(qs, qoff, packed["scene_min"], packed["scene_max"],
-                                                   bvh["batch_size"], schedule=True)
-                     if scheduled else None)
-            if events:
-                events[2].record()
-            out = _C.query_knn_ragged(
-                packed["node_aabbs"], packed["sorted_indices"], bvh["batch_offsets"], packed["node_offsets"],
-                qs, qoff, order, bvh["batch_size"], D, k, accel=bvh._aux["accel"],
-                total_points=bvh._aux["host_offsets"][-1])
-        else:
-            one = kind == "single"
-            qb = qs.unsqueeze(0) if one else qs
-            smin = bvh["scene_min"].unsqueeze(0) if one else bvh["scene_min"]
-            smax = bvh["scene_max"].unsqueeze(0) if one else bvh["scene_max"]
-            nodes = bvh["node_aabbs"].unsqueeze(0) if one else bvh["node_aabbs"]
-            sidx = bvh["sorted_indices"].unsqueeze(0) if one else bvh["sorted_indices"]
-            if scheduled:
-                order = _C.morton_sort_queries_narrow(qb, smin, smax, schedule=True)
-            if events:
-                events[2].record()
-            if scheduled:
-                out = _C.query_knn_batched_cached_bounds_ordered(
-                    nodes, sidx, qb, order, bvh["num_leaves"], bvh["num_real_nodes"], D, k,
-                    accel=bvh._aux["accel"])
-            else:
-                out = _C.query_knn_batched_cached_bounds(
-                    nodes, sidx, qb, bvh["num_leaves"], bvh["num_real_nodes"], D, k, accel=bvh._aux["accel"])
+        out = query_phases(kind, bvh, qs, qoff, k, events[2].record if events else lambda: None)
         if events:
             events[3].record()
         return bvh, out
@@ -699,7 +717,7 @@ def main() -> int:
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32",
-        "data": "synthetic (seeded torch CPU generator, BASELINE config shapes)",
+        "data": "synthetic (seeded torch CPU generator, the config's shapes)",
         "config": {
             "workload": CONFIGS[args.config],
             "config_id": args.config,
@@ -711,15 +729,16 @@ def main() -> int:
         "build_ms": build_ms,
         "query_ms": query_ms,
         "query_sort_ms": sort_ms,
-        "query_sort_what": ("traversal schedule: stable 2-pass radix sort on the top 16 bits of Hilbert keys"
-                            if scheduled else "none: at most SCHEDULE_MIN_QUERIES queries run in input order"),
+        "query_sort_what": order_what,
         "traversal_ms": trav_ms,
         "traversal_implicit_tree_ms": implicit_ms,
         "queries_per_s_excl_build": total_q / (query_ms * 1e-3) if query_ms > 0 else None,
         "build_hbm_frac_algorithmic": (b_bytes / (build_ms * 1e-3) / 1e9) / HBM_PEAK_GBS,
         "query_sort_hbm_frac_algorithmic": ((s_bytes / (sort_ms * 1e-3) / 1e9) / HBM_PEAK_GBS
-                                            if sort_ms and scheduled else None),
-        "query_sort_bytes_formula": "Q(4D+40): queries read, 4-B keys, 2 passes x 16 B, 4-B order",
+                                            if sort_ms and order != "input" else None),
+        "query_sort_bytes_formula": ("Q(4D+56): queries read, 4-B keys, 2 passes x 16 B, 16 B within tiles, 4-B order"
+                                     if order == "fine" else
+                                     "Q(4D+40): queries read, 4-B keys, 2 passes x 16 B, 4-B order"),
         "query_sort_full_ms": full_sort_ms,
         "query_sort_full_what": "reference binding morton_sort_queries_narrow: 30/32-bit Morton keys, 4 passes",
         "query_sort_full_hbm_frac_algorithmic": ((full_sort_bytes / (full_sort_ms * 1e-3) / 1e9) / HBM_PEAK_GBS

@@ -7,7 +7,11 @@ import subprocess
 import sys
 from pathlib import Path
 
+import pytest
+import torch
+
 import bench
+from torchbvh_amd import _handles, _native, _query
 
 ROOT = Path(__file__).resolve().parents[1]
 
@@ -60,3 +64,52 @@ def test_more_than_one_gpu_is_refused():
                        capture_output=True, text=True, cwd=ROOT, timeout=120)
     assert r.returncode != 0
     assert "one GPU" in (r.stdout + r.stderr)
+
+
+@pytest.mark.parametrize("kind,rows,order", [("single", 1 << 17, "input"), ("single", (1 << 17) + 1, "schedule"),
+                                             ("single", 1 << 20, "fine"), ("batched", 1 << 20, "schedule"),
+                                             ("batched", 1 << 21, "fine"), ("ragged", 1 << 21, "schedule")])
+def test_timed_query_calls_are_those_of_query_knn(monkeypatch, kind, rows, order):
+    """The timed step makes the binding calls of ``tb.query_knn``, with the same arguments."""
+    made = []
+
+    def record(name):
+        def call(*args, **kwargs):
+            made.append((name, [tuple(a.shape) if isinstance(a, torch.Tensor) else a for a in args], kwargs))
+            found = torch.zeros(1, dtype=torch.int64)
+            return (found, found) if name.startswith("query") else found
+        return staticmethod(call)
+
+    for name in ("morton_sort_queries_narrow", "morton_sort_queries_ragged", "safe_offsets", "query_knn_ragged",
+                 "query_knn_batched_cached_bounds", "query_knn_batched_cached_bounds_ordered"):
+        monkeypatch.setattr(_native._NativeOps, name, record(name))
+    for check in ("check_cuda_f32", "check_source_points"):
+        monkeypatch.setattr(_query, check, lambda *a, **kw: None)
+
+    class Read:
+        def __init__(self, *a, **kw):
+            pass
+
+        def values(self):
+            return [0, rows // 2, rows]
+
+    monkeypatch.setattr(_query, "OffsetsRead", Read)
+    lead = {"single": (), "batched": (2,), "ragged": ()}[kind]
+    n, k = 64, 16
+    tree = {"node_aabbs": torch.zeros((*lead, 2 * n - 1, 6)), "sorted_indices": torch.zeros((*lead, n), dtype=torch.int64),
+            "scene_min": torch.zeros((*lead, 3)), "scene_max": torch.zeros((*lead, 3)), "num_leaves": n,
+            "num_real_nodes": 2 * n - 1, "dim": 3, "batch_size": 2, "batch_offsets": torch.tensor([0, 32, 64])}
+    aux = {"accel": "the accel", "host_offsets": [0, 32, 64],
+           "packed": {**tree, "node_offsets": torch.zeros(3, dtype=torch.int64)}}
+    handle = {"single": _handles.BVHHandle, "batched": _handles.BatchedBVHHandle,
+              "ragged": lambda data, aux: _handles.RaggedBVHHandle(data, [], aux)}[kind](tree, aux)
+    queries = torch.zeros((2, rows // 2, 3) if kind == "batched" else (rows, 3))
+    offsets = torch.tensor([0, rows // 2, rows])
+    query = {"single": _query._query_knn_single, "batched": _query._query_knn_batched,
+             "ragged": _query._query_knn_ragged}[kind]
+    query(handle, queries, *((offsets, k) if kind == "ragged" else (k,)))
+    public, made[:] = list(made), []
+    bench.query_phases(kind, handle, queries, offsets, k, lambda: made.append("between"))
+    assert bench.query_order(kind, 2 if kind == "batched" else 1, rows, k) == order
+    assert made.pop(-2) == "between"
+    assert made == public
