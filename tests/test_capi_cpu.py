@@ -422,3 +422,21 @@ def test_build_noalloc_argument_errors():
     assert size.value > 64 << 20
     assert L.tbvh_build_with_accel_noalloc(FAKE, 1, 1 << 23, 3, *outs, FAKE, None) == 2
     assert "scratch array holds 67108864" in _err(L)
+
+
+def test_ragged_trim_cuts_at_the_librarys_node_counts(monkeypatch):
+    """The node arrays of a bounded ragged build are cut by tbvh_real_node_count."""
+    import torch
+
+    from torchbvh_amd import _native
+
+    counts = [1, 2, 5, 17]
+    names = ("node_aabbs", "left_child_mem", "right_child_mem", "mem_to_leaf")
+    packed = _native._NativeOps.trim_ragged_build({**{k: torch.zeros((99, 2)) for k in names}, "accel": None}, counts)
+    expected = [0]
+    for c in counts:
+        expected.append(expected[-1] + int(_native.load().tbvh_real_node_count(c)))
+    assert packed["host_node_offsets"] == expected and all(len(packed[k]) == expected[-1] for k in names)
+    monkeypatch.setattr(_native.load(), "tbvh_real_node_count", lambda n: 3 * n)
+    packed = _native._NativeOps.trim_ragged_build({**{k: torch.zeros((99, 2)) for k in names}, "accel": None}, counts)
+    assert packed["host_node_offsets"] == [0, 3, 9, 24, 75]

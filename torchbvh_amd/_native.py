@@ -726,10 +726,10 @@ class _NativeOps:
     def trim_ragged_build(packed: dict, counts: list[int]) -> dict:
         """`packed` with its node arrays cut to the nodes that clouds of these
         sizes have and the clouds' node offsets added; records the accel."""
+        nodes = load().tbvh_real_node_count
         host_node_offsets = [0]
         for c in counts:
-            level = (c - 1).bit_length()
-            host_node_offsets.append(host_node_offsets[-1] + 2 * c - 1 + bin((1 << level) - c).count("1"))
+            host_node_offsets.append(host_node_offsets[-1] + nodes(c))
         total = host_node_offsets[-1]
         for key in ("node_aabbs", "left_child_mem", "right_child_mem", "mem_to_leaf"):
             packed[key] = packed[key][:total]
