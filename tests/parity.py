@@ -119,3 +119,37 @@ def unit_direction_points(dim: int) -> np.ndarray:
     eye = np.eye(dim, dtype=np.float32)
     dirs = np.concatenate([np.stack((eye[d], -eye[d])) for d in range(dim)])
     return np.concatenate((np.repeat(dirs, 4, axis=0), 3.0 * dirs)).astype(np.float32)
+
+
+ROUTES = ("dispatched", "tail", "plain")
+
+
+def force_route(monkeypatch, route: str) -> None:
+    """Accel k-NN below the cell-block search's sizes as dispatched (one wave
+    per query for few queries), by the traversal that gives up its last
+    queries ("tail"), or by the whole traversal ("plain")."""
+    from torchbvh_amd import _native
+
+    if route == "dispatched":
+        return
+    for name in ("WAVE_MAX_QUERIES", "WAVE_MAX_QUERIES_2D", "WAVE_MAX_QUERIES_2D_LARGE"):
+        monkeypatch.setattr(_native, name, 0)
+    if route == "tail":
+        return
+    L = _native.load()
+
+    def batched(accel, nodes, real, q, order, B, M, n, D, k, spatial, source, cols, idx, dist, rows, ws, size, stream):
+        if source is not None:
+            return L.tbvh_knn_accel_positions(accel, q, order, B, M, n, D, k, source, cols, idx, dist, rows, stream)
+        plain = L.tbvh_knn_accel_spatial if spatial else L.tbvh_knn_accel
+        return plain(accel, q, order, B, M, n, D, k, idx, dist, stream)
+
+    def ragged(accel, nodes, node_offsets, offsets, total, q, q_offsets, order, B, T, D, k, source, cols, idx, dist,
+               rows, ws, size, stream):
+        common = (accel, offsets, total, q, q_offsets, order, B, T, D, k)
+        if source is not None:
+            return L.tbvh_knn_accel_ragged_positions(*common, source, cols, idx, dist, rows, stream)
+        return L.tbvh_knn_accel_ragged(*common, idx, dist, stream)
+
+    monkeypatch.setattr(L, "tbvh_knn_accel_tail", batched)
+    monkeypatch.setattr(L, "tbvh_knn_accel_ragged_tail", ragged)

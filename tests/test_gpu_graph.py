@@ -14,7 +14,8 @@ import pytest
 import torch
 
 import torchbvh_amd as tb
-from torchbvh_amd import _query
+from parity import ROUTES, force_route
+from torchbvh_amd import _native, _query
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
@@ -25,10 +26,16 @@ def cloud(seed: int, n: int, dim: int) -> torch.Tensor:
     return torch.rand((n, dim), generator=g).to(DEV)
 
 
+@pytest.mark.parametrize("route", [*ROUTES, "cells"])
 @pytest.mark.parametrize("dim,k", [(3, 16), (2, 8)])
-def test_build_and_knn_replay_under_graph_capture(dim, k, monkeypatch):
+def test_build_and_knn_replay_under_graph_capture(dim, k, route, monkeypatch):
+    force_route(monkeypatch, "dispatched" if route == "cells" else route)
     monkeypatch.setattr(_query, "SCHEDULE_MIN_QUERIES", 0)  # capture the schedule sort too
     n, m = 60_000, 20_000
+    if route == "cells":  # the cell-block search, and the finer schedule
+        monkeypatch.setattr(_query, "FINE_MIN_QUERIES", 0)
+        m = 140_000
+        assert _native._grid_workspace_size(1, m, n, dim, k) > 0
     p = cloud(1, n, dim)
     q = cloud(2, m, dim)
 

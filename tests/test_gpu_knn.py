@@ -17,6 +17,7 @@ import torchbvh_amd as tb
 from parity import (
     assert_same_f32,
     assert_same_int,
+    force_route,
     knn_pathological_clouds,
     unit_direction_points,
 )
@@ -36,6 +37,13 @@ def schedule_mode(request, monkeypatch):
     if request.param == "scheduled":
         monkeypatch.setattr(_query, "SCHEDULE_MIN_QUERIES", 0)
     return request.param
+
+
+@pytest.fixture(autouse=True, params=["dispatched", "plain"])
+def route(request, monkeypatch):
+    force_route(monkeypatch, request.param)
+
+
 DEV = torch.device("cuda")
 DIST_RTOL = 1e-6  # contractual tolerance; checked in addition to bit equality
 

@@ -22,11 +22,18 @@ import torch
 
 import oracle
 import torchbvh_amd as tb
-from parity import assert_same_f32, assert_same_int
+from parity import ROUTES, assert_same_f32, assert_same_int, force_route
 from torchbvh_amd._native import _C
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
+
+
+@pytest.fixture(autouse=True, params=ROUTES)
+def route(request, monkeypatch):
+    force_route(monkeypatch, request.param)
+
+
 INF, NAN = np.float32(np.inf), np.float32(np.nan)
 
 

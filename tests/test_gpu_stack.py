@@ -16,10 +16,18 @@ import torch
 
 import oracle
 import torchbvh_amd as tb
-from parity import assert_same_f32, assert_same_int
+from parity import ROUTES, assert_same_f32, assert_same_int, force_route
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
+
+
+@pytest.fixture(autouse=True, params=ROUTES)
+def route(request, monkeypatch):
+    """Every case by each search: these few queries take one wave each as
+    dispatched, and only the whole traversal fills its rings and resumes."""
+    force_route(monkeypatch, request.param)
+    return request.param
 
 
 def dev(a) -> torch.Tensor:

@@ -209,3 +209,76 @@ def test_given_up_queries_among_nan_points(layout, k):
     assert (np.diff(np.sort(idx, axis=1), axis=1) > 0).all()
     assert (np.diff(d2, axis=1) >= 0).all()
     assert np.array_equal(d2, oracle.pair_distances(pts, q, idx))
+
+
+def _marks(ws, total_q, dim, k, grid):
+    """The work-groups whose traversal gave queries up, from a call's workspace
+    (knn.hip: set_tail, grid_layout)."""
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    groups = -(-(-(-total_q // 64)) // 8) * 8
+    if not grid:
+        masks = ws[: groups * 8].view(torch.int64).cpu()
+        return int((masks[: total_q // 64] != 0).sum())
+    seg = -(-(groups // 8) // 64) * 64
+    list2 = ws.numel() - up(total_q * 4) - up(512 * seg * 4)
+    list1 = list2 - up(512 * seg * 4)
+    counts = ws[list1 - 2 * 512 * 32 * 4: list1].view(torch.int32).view(2, 512, 32)[:, :, 0].cpu()
+    two_passes = dim == 3 and k in (8, 16)
+    masks = ws[list1 if two_passes else list2:][: groups * 8].view(torch.int64).cpu()
+    b = torch.arange(groups)
+    sub, chunk = b % 8 * 64 + b // 8 % 64, b // 8 // 64
+    return int((masks[chunk * 64 < counts[1 if two_passes else 0][sub]] != 0).sum())
+
+
+@pytest.mark.parametrize("k", [8, 16, 32])
+@pytest.mark.parametrize("layout", ["batched", "rows", "ordered", "spatial", "ragged", "grid", "routed", "routed grid"])
+def test_queries_are_given_up_in_every_layout(monkeypatch, layout, k):
+    """The tail runs in each of them, and the rows are the whole traversal's."""
+    L, p, used = _native.load(), _native._ptr, []
+
+    def in_kept_workspace(entry):
+        def call(*args):  # (..., workspace, size, stream)
+            used.append(torch.zeros(args[-2], dtype=torch.uint8, device="cuda"))
+            return entry(*args[:-3], p(used[-1]), *args[-2:])
+        return call
+
+    for name in LIMITS:
+        monkeypatch.setattr(_native, name, 0)
+    for name in ("tail", "ragged_tail", "routed_tail", "grid", "routed_grid_spatial"):
+        monkeypatch.setattr(L, f"tbvh_knn_accel_{name}", in_kept_workspace(getattr(L, f"tbvh_knn_accel_{name}")))
+    grid = "grid" in layout
+    m = 134_000 if grid else 30_000
+    q = _centre(m, 3, 3)[None]
+    order = torch.randperm(m, generator=torch.Generator().manual_seed(1)).cuda()[None].contiguous()
+    idx, dist = torch.empty((m, k), dtype=torch.int64, device="cuda"), torch.empty((m, k), device="cuda")
+    stream = _native._stream(q.device)
+    if layout == "ragged":
+        off, qoff = torch.tensor([0, 15_000, 33_000], device="cuda"), torch.tensor([0, 9_999, m], device="cuda")
+        bvh = tb.build_bvh(_shell(33_000, 3, 1), batch_offsets=off)
+        got = tb.query_knn(bvh, q[0], k, query_offsets=qoff)
+        _native._check(L.tbvh_knn_accel_ragged(p(bvh._aux["accel"]), p(off), 33_000, p(q), p(qoff), None, 2, m, 3, k,
+                                               p(idx), p(dist), stream))
+    elif layout.startswith("routed"):
+        routes = torch.arange(m, device="cuda")[None] % 3 == 0
+        t, f = (_C.build_bvh_batched_cooperative(c[None], with_accel=True)
+                for c in (_shell(33_000, 3, 1), 1.5 * _shell(34_000, 3, 2)))
+        got = _C.query_knn_routed_batched_cached_bounds_spatial(
+            t["node_aabbs"], t["sorted_indices"], f["node_aabbs"], f["sorted_indices"], q, routes, order,
+            t["num_leaves"], t["num_real_nodes"], f["num_leaves"], f["num_real_nodes"], 3, k)
+        _native._check(L.tbvh_knn_accel_routed_spatial(p(t["accel"]), p(f["accel"]), p(q), p(routes), p(order), 1, m,
+                                                       33_000, 34_000, 3, k, p(idx), p(dist), stream))
+    else:
+        pts = _shell(33_000, 3, 1)[None]
+        d = _C.build_bvh_batched_cooperative(pts, with_accel=True)
+        tree, sizes = (d["node_aabbs"], d["sorted_indices"], q), (33_000, d["num_real_nodes"], 3, k)
+        plain = L.tbvh_knn_accel
+        if layout in ("ordered", "spatial"):
+            call = getattr(_C, f"query_knn_batched_cached_bounds_{layout}")
+            got = call(*tree, order, *sizes)
+            plain = L.tbvh_knn_accel_spatial if layout == "spatial" else plain
+        else:
+            got = _C.query_knn_batched_cached_bounds(*tree, *sizes, source_points=pts if layout == "rows" else None)
+        _native._check(plain(p(d["accel"]), p(q), p(order) if layout in ("ordered", "spatial") else None, 1, m, 33_000,
+                             3, k, p(idx), p(dist), stream))
+    assert torch.equal(got[0].reshape(m, k), idx) and torch.equal(got[1].reshape(m, k), dist)
+    assert len(used) == 1 and _marks(used[0], m, 3, k, grid) > 100
