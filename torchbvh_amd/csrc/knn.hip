@@ -808,7 +808,7 @@ __device__ __forceinline__ void knn_query(const KnnArgs& a) {
     if (gid >= a.total_q) return;
     const QueryLoc in = locate<kOrdered, kRagged, kRouted, kAccel>(a, gid);
     if (in.row < 0) return;
-    const bool tail = kAccel && a.tail_masks != nullptr;
+    const bool tail = kAccel && D == 3 && a.tail_masks != nullptr;
 
     float q[D];
 #pragma unroll

@@ -357,7 +357,7 @@ __global__ __launch_bounds__(kWave) void knn_wave_kernel(KnnArgs a) {
 // or by its neighbours, go to different work-groups (four lanes per work-group
 // read the marks in 5 us instead of 6 at 18,400 work-groups, but the routed
 // search of 357,000 queries of surface clouds went 1.7 -> 4.4 ms).
-template <int D, int K, bool kOrdered, bool kRagged, bool kRouted>
+template <int K, bool kOrdered, bool kRagged, bool kRouted>
 __global__ __launch_bounds__(kWave) void knn_tail_kernel(KnnArgs a, int groups) {
     const int stride = static_cast<int>(gridDim.x) / kWave;
     const int slot = static_cast<int>(blockIdx.x) % kWave;
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(kWave) void knn_tail_kernel(KnnArgs a, int groups) 
                 gid = a.fb_list[sub * a.fb_seg + static_cast<int64_t>(rest / kGridSubLists) * kKnnBlock + slot];
             }
             const QueryLoc l = locate<kOrdered, kRagged, kRouted, false>(a, gid);
-            if (l.row >= 0) wave_search<D, K, 0>(a, l, a.tail_bounds[gid]);
+            if (l.row >= 0) wave_search<3, K, 0>(a, l, a.tail_bounds[gid]);
         }
     }
 }
@@ -422,37 +422,33 @@ hipError_t launch_wave_k(const KnnArgs& a, int K, bool ragged, hipStream_t strea
     return hipGetLastError();
 }
 
-template <int D, int K>
+template <int K>
 void launch_tail(const KnnArgs& a, bool ragged, hipStream_t stream) {
     // The traversal's grid (knn.hip launch_dk); 64 work-groups per stride.
     const int64_t tiles = (a.total_q + kKnnBlock - 1) / kKnnBlock;
     const int groups = static_cast<int>((tiles + kXcds - 1) / kXcds * kXcds);
     const unsigned grid = static_cast<unsigned>(std::min((groups + kWave - 1) / kWave, 128) * kWave);
     const bool ordered = a.order != nullptr;
-    if (a.routes != nullptr) knn_tail_kernel<D, K, true, false, true><<<grid, kWave, 0, stream>>>(a, groups);
-    else if (ragged && ordered) knn_tail_kernel<D, K, true, true, false><<<grid, kWave, 0, stream>>>(a, groups);
-    else if (ragged) knn_tail_kernel<D, K, false, true, false><<<grid, kWave, 0, stream>>>(a, groups);
-    else if (ordered) knn_tail_kernel<D, K, true, false, false><<<grid, kWave, 0, stream>>>(a, groups);
-    else knn_tail_kernel<D, K, false, false, false><<<grid, kWave, 0, stream>>>(a, groups);
-}
-
-template <int D>
-hipError_t launch_tail_k(const KnnArgs& a, int K, bool ragged, hipStream_t stream) {
-    switch (K) {
-        case 4: launch_tail<D, 4>(a, ragged, stream); break;
-        case 8: launch_tail<D, 8>(a, ragged, stream); break;
-        case 16: launch_tail<D, 16>(a, ragged, stream); break;
-        case 32: launch_tail<D, 32>(a, ragged, stream); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    if (a.routes != nullptr) knn_tail_kernel<K, true, false, true><<<grid, kWave, 0, stream>>>(a, groups);
+    else if (ragged && ordered) knn_tail_kernel<K, true, true, false><<<grid, kWave, 0, stream>>>(a, groups);
+    else if (ragged) knn_tail_kernel<K, false, true, false><<<grid, kWave, 0, stream>>>(a, groups);
+    else if (ordered) knn_tail_kernel<K, true, false, false><<<grid, kWave, 0, stream>>>(a, groups);
+    else knn_tail_kernel<K, false, false, false><<<grid, kWave, 0, stream>>>(a, groups);
 }
 
 }  // namespace
 
 hipError_t launch_knn_tail(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream) {
     if (a.total_q == 0) return hipSuccess;
-    return D == 3 ? launch_tail_k<3>(a, K, ragged, stream) : launch_tail_k<2>(a, K, ragged, stream);
+    if (D != 3) return hipErrorInvalidValue;  // tail_workspace_bytes
+    switch (K) {
+        case 4: launch_tail<4>(a, ragged, stream); break;
+        case 8: launch_tail<8>(a, ragged, stream); break;
+        case 16: launch_tail<16>(a, ragged, stream); break;
+        case 32: launch_tail<32>(a, ragged, stream); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_knn_wave(const KnnArgs& a, int D, int K, bool ragged, hipStream_t stream) {

@@ -326,8 +326,8 @@ template <int D>
 void launch_d(const float* rows, const Segment* segs, int64_t S, UniformPlan plan, int64_t max_n, float* scene_min,
               float* scene_max, bool bounds, float seed_lo, float seed_hi, SortBits bits, int64_t* order,
               uint32_t* sorted_keys, hipStream_t stream) {
-    // Up to 4 keys per thread (48 kB of LDS) to 4,096 rows, else up to 12
-    // (112 kB).  At 16 keys per thread (16,384 rows) this kernel measured
+    // Up to 4 keys per thread (51 kB of LDS) to 4,096 rows, else up to 12
+    // (133 kB).  At 16 keys per thread (16,384 rows) the stable passes measured
     // slower than the general sequence (full build 130.6 against 121.5 us at
     // 16,384 points), at 10,000 points faster (107.4 against 120.5 us).
     if (max_n <= 4 * kSmallThreads) {

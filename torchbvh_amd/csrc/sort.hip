@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kScanThreads) void tile_scan_kernel(const uint32_t*
 }
 
 // kInline: the tile sums its cloud's digit counts itself (tile_hist, tile-
-// major), and no scan is launched (sort_sums_inline).
+// major), and no scan is launched (sort_tstride).
 template <bool kFirst, bool kLast, bool kInline>
 __global__ __launch_bounds__(kThreads) void scatter_kernel(const Segment* __restrict__ segs, int S,
                                                            SortPass pass) {
