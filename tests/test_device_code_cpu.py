@@ -179,3 +179,10 @@ def test_accel_traversal_keeps_its_occupancy(assembly, dim, k, compact, waves):
     for ordered in (0, 1):  # (D, K, ordered, ragged, routed, compact)
         used = registers[(dim, k, ordered, 0, 0, compact)]
         assert 512 // (-(-used // 8) * 8) >= waves, used
+
+
+def test_schedule_refinement_fits_two_work_groups_per_cu(assembly):
+    """Work-groups of 16 waves: eight waves per SIMD, 64 registers."""
+    body = re.search(r"\.amdhsa_kernel \S*refine_kernel\S*\n(.*?)\.end_amdhsa_kernel", assembly["small.hip"], re.S).group(1)
+    assert int(re.search(r"\.amdhsa_next_free_vgpr (\d+)", body).group(1)) <= 64
+    assert int(re.search(r"\.amdhsa_private_segment_fixed_size (\d+)", body).group(1)) == 0

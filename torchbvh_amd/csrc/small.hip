@@ -343,7 +343,9 @@ void launch_d(const float* rows, const Segment* segs, int64_t S, UniformPlan pla
 // order of all their bits (nearly), for a schedule, whose order changes no
 // result.  Bins over the tile's key range and sub-bins as in the small sort, by
 // the key's place in the range.  One read and one write of 8 bytes a row: 8 us at
-// 1M rows, 24 at 4M, where two more passes of the global sort took 32 and 66.
+// 1M rows, 18 at 4M, where two more passes of the global sort took 32 and 66.
+// The rows wait in LDS: in registers they took the kernel past 64, one
+// work-group per CU in place of two (24 us at 4M rows).
 //
 // Every call gives the same order: among points with a NaN coordinate a search's
 // rows depend on which queries share a wave.  Rows of a slot in the order they
@@ -369,12 +371,12 @@ __global__ __launch_bounds__(kSmallThreads) void refine_kernel(const Segment* __
     if (lt >= g.tiles) return;  // surplus tile
     const int64_t row0 = g.start + static_cast<int64_t>(lt) * kSortTile;
     const int count = min(kSortTile, g.n - lt * kSortTile);
-    uint32_t key[kItems], val[kItems];
+    uint32_t key[kItems];
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
         const int j = i * kSmallThreads + threadIdx.x;
         key[i] = keys[row0 + (j < count ? j : 0)];
-        val[i] = vals[row0 + (j < count ? j : 0)];
+        s_vals[j] = vals[row0 + (j < count ? j : 0)];
     }
     const uint32_t low = (1u << (key_bits - 16)) - 1u;
     const uint32_t base = keys[row0] & ~low;
@@ -409,36 +411,39 @@ __global__ __launch_bounds__(kSmallThreads) void refine_kernel(const Segment* __
     for (int i = 0; i < kItems; ++i) {
         if (i * kSmallThreads + threadIdx.x < count) most = max(most, at[i] >> 16);
     }
-    if (__syncthreads_or(most >= kMostInBin)) {
-        // Many rows of one key or nearly: the tile stays as it is.
+    uint16_t* rows16 = reinterpret_cast<uint16_t*>(bins);
+    // With many rows of one key or nearly, the tile stays as it is.
+    const bool sorted = !__syncthreads_or(most >= kMostInBin);
+    if (sorted) {
+        scan_halves<kItems>(sub, s_scan);
 #pragma unroll
         for (int i = 0; i < kItems; ++i) {
             const int j = i * kSmallThreads + threadIdx.x;
-            if (j < count) order[row0 + j] = static_cast<int64_t>(val[i]);
+            if (j < count) rows16[read_half(sub, at[i] & 0xffffu) + (at[i] >> 16)] = static_cast<uint16_t>(j);
         }
-        return;
-    }
-    scan_halves<kItems>(sub, s_scan);
-    uint16_t* arrivals = reinterpret_cast<uint16_t*>(bins);
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kItems; ++i) {
-        const int j = i * kSmallThreads + threadIdx.x;
-        if (j < count) arrivals[read_half(sub, at[i] & 0xffffu) + (at[i] >> 16)] = static_cast<uint16_t>(j);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kItems; ++i) {
-        const int j = i * kSmallThreads + threadIdx.x;
-        if (j < count) {
-            const uint32_t slot = at[i] & 0xffffu;
-            const uint32_t first = read_half(sub, slot), end = read_half(sub, slot + 1);
-            uint32_t place = first;
-            for (uint32_t o = first; o < end; ++o) place += arrivals[o] < j ? 1u : 0u;
-            s_vals[place] = val[i];
+        for (int i = 0; i < kItems; ++i) {
+            const int j = i * kSmallThreads + threadIdx.x;
+            if (j < count) {
+                const uint32_t slot = at[i] & 0xffffu;
+                const uint32_t first = read_half(sub, slot), end = read_half(sub, slot + 1);
+                uint32_t place = first;
+                for (uint32_t o = first; o < end; ++o) place += rows16[o] < j ? 1u : 0u;
+                at[i] = place;
+            }
         }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            const int j = i * kSmallThreads + threadIdx.x;
+            if (j < count) rows16[at[i]] = static_cast<uint16_t>(j);
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    for (int j = threadIdx.x; j < count; j += kSmallThreads) order[row0 + j] = static_cast<int64_t>(s_vals[j]);
+    for (int j = threadIdx.x; j < count; j += kSmallThreads) {
+        order[row0 + j] = static_cast<int64_t>(s_vals[sorted ? rows16[j] : j]);
+    }
 }
 
 }  // namespace
